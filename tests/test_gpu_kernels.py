@@ -258,6 +258,46 @@ def test_gemv_tq_bit_exact(bits, kb, rows, K, pair, m, strips):
     gemv_check(to_dev(tq), tq, rows, K, fmt, bits, kb, x, pair, strips)
 
 
+# Enough (strip, pass) workgroups for the MFMA tiles: every codec, ragged row and activation tiles (the
+# last workgroup nearly empty), k short of a slice and past one, strip sub-ranges, pairs, accumulate;
+# 64-row workgroups from 769 of 32 rows (m = 520 at 48 row blocks)
+GEMM_CASES = [(O.FMT_Q4_K, 32, 1000, 512, False, 129, None), (O.FMT_Q4_K, 16, 440, 256, True, 145, (1, 27)),
+              (O.FMT_Q6_K, 16, 520, 768, False, 241, (3, 33)), (O.FMT_Q8_0, 32, 1160, 256, False, 100, None),
+              (O.FMT_Q8_0, 16, 240, 512, True, 260, None), (O.FMT_Q5_1, 32, 480, 256, False, 241, None),
+              (O.FMT_Q5_1, 16, 1040, 256, False, 111, None), ((4, 32), 32, 900, 1056, False, 127, None),
+              ((4, 16), 16, 1800, 80, False, 65, None), ((5, 32), 32, 700, 320, True, 91, (2, 44)),
+              ((5, 16), 16, 2560, 176, False, 45, (0, 157)), ((8, 32), 32, 28700, 32, False, 5, None),
+              ((8, 16), 16, 400, 640, False, 289, None), ((8, 32), 32, 6100, 160, False, 520, None),
+              ((5, 16), 16, 6100, 272, True, 260, None), (O.FMT_Q6_K, 16, 6100, 256, False, 520, None)]
+
+
+@pytest.mark.parametrize("fmt,kb,rows,K,pair,m,strips", GEMM_CASES)
+def test_gemv_many_rows_bit_exact(fmt, kb, rows, K, pair, m, strips):
+    """trk_gemv of many activation rows against the oracle's gemm_tq_rows, written and accumulated,
+    into a y wider than the matrix: the bits of the chain, nothing outside the strip range."""
+    say(f"gemm fmt={fmt} kb={kb} rows={rows} K={K} pair={pair} m={m} strips={strips}")
+    if isinstance(fmt, tuple):
+        bits, code = fmt[0], (fmt[0] << 8) | fmt[1]
+        raw = tq = random_tq(11 + bits + m, rows, K, bits, kb)
+    else:
+        code, raw = fmt, O.gen_gguf(fmt, 3, 60 + fmt + kb, rows, K)
+        tq, bits = O.gguf_to_tq(fmt, raw, rows, K, kb)
+    q, s, su = act_rows(O.gen_normal(5, 70 + m, m * K, 1.0).reshape(m, K), kb, pair)
+    nstrips = (rows + 15) // 16
+    s0, s1 = strips or (0, nstrips)
+    assert (s1 - s0) * ((q.shape[0] + 3) // 4) >= 7 * 256  # the tiles' range
+    c0, c1 = 16 * s0, 16 * s1 if isinstance(fmt, tuple) else min(16 * s1, rows)
+    ldy = 16 * nstrips + 3
+    base = (np.arange(m * ldy, dtype=np.float32).reshape(m, ldy) % 97) * 0.25
+    for acc in (False, True):
+        want = O.gemv_tq(tq, K, bits, kb, 16 * nstrips, q, s, su, pair=pair, y=base.copy(),
+                         rows=np.arange(m, dtype=np.uint32), accumulate=acc, s0=s0, s1=s1, ldy=ldy)
+        got = host(trmoe.gemv(to_dev(raw), rows, K, code, 0, 1, kb, to_dev(q), to_dev(s), to_dev(su), pair=pair,
+                              y=to_dev(base.copy()), ldy=ldy, accumulate=acc, s0=s0, s1=s1))
+        assert np.array_equal(got[:, c0:c1].view(np.uint32), want[:, c0:c1].view(np.uint32)), acc
+        assert np.array_equal(got[:, :c0], base[:, :c0]) and np.array_equal(got[:, c1:], base[:, c1:]), acc
+
+
 @pytest.mark.parametrize("m", [1, 70, 300, 512])
 def test_designed_rounding_orders(m):
     """The designed cases that pin the oracle's f32 orders (test_oracle.py: test_gemv_epilogue_order,

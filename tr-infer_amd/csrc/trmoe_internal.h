@@ -172,6 +172,10 @@ hipError_t launch_batch_combine(const Workspace& ws, uint32_t m, float* out, int
 hipError_t launch_gemv(const Mat& w, uint32_t item, uint32_t s0, uint32_t s1, uint32_t kb, const int8_t* q,
                        const float* s, const int32_t* su, uint32_t m, int pair, float* y, uint32_t ldy,
                        const uint32_t* rows, int accumulate, hipStream_t st);
+// the same for many activation rows without a row map, as MFMA tiles (k_gemm.hip)
+hipError_t launch_gemm(const Mat& w, uint32_t item, uint32_t s0, uint32_t s1, uint32_t kb, const int8_t* q,
+                       const float* s, const int32_t* su, uint32_t m, int pair, float* y, uint32_t ldy,
+                       int accumulate, hipStream_t st);
 // the layer on TQ experts (k_tq.hip): gate/up into h [rows][2F], SwiGLU + quantisation + fold,
 // down into yent, and (decode) the slot-order combine
 hipError_t launch_tq_gateup(const Mat& gate, const Mat& up, const Mat& sh_gate, const Mat& sh_up, const Workspace& ws,
