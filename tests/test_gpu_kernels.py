@@ -258,6 +258,23 @@ def test_gemv_tq_bit_exact(bits, kb, rows, K, pair, m, strips):
     gemv_check(to_dev(tq), tq, rows, K, fmt, bits, kb, x, pair, strips)
 
 
+# Few TQ rows take four rows per workgroup (rows x passes of four up to 2048), more a strip per workgroup:
+# both sides of the line, slices of 256 blocks (128 from three activation rows) and one block past them
+GEMV_QUAD_CASES = [(4, 32, 2048, 320, False, 1, None), (4, 32, 2064, 320, False, 3, None),
+                   (5, 32, 2064, 352, True, 1, None), (8, 32, 2064, 96, False, 2, None),
+                   (4, 16, 2080, 80, False, 4, (1, 130)), (5, 16, 512, 4112, True, 1, (3, 32)),
+                   (8, 32, 320, 10240, True, 1, None), (8, 32, 64, 4128, False, 4, None),
+                   (8, 16, 48, 2064, False, 3, (0, 2)), (4, 16, 1024, 4096, False, 8, None)]
+
+
+@pytest.mark.parametrize("bits,kb,rows,K,pair,m,strips", GEMV_QUAD_CASES)
+def test_gemv_few_rows_bit_exact(bits, kb, rows, K, pair, m, strips):
+    say(f"gemv quads bits={bits} kb={kb} rows={rows} K={K} pair={pair} m={m} strips={strips}")
+    tq = random_tq(9 + bits + kb + m, rows, K, bits, kb)
+    x = O.gen_normal(4, 80 + m, m * K, 1.0).reshape(m, K)
+    gemv_check(to_dev(tq), tq, rows, K, (bits << 8) | kb, bits, kb, x, pair, strips)
+
+
 # Enough (strip, pass) workgroups for the MFMA tiles: every codec, ragged row and activation tiles (the
 # last workgroup nearly empty), k short of a slice and past one, strip sub-ranges, pairs, accumulate;
 # 64-row workgroups from 769 of 32 rows (m = 520 at 48 row blocks)

@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvArgs g) {
         if constexpr (TQ) {
             const uint32_t u = gi + 16 * k, sl = u % NSTR, j = u / NSTR;
             const uint32_t st = row0 / 16 + sl, stc = st < g.r_hi / 16 ? st : g.r_hi / 16 - 1;
-            gv_load_tq<GK, KB>(wi, g.w + (size_t)stc * g.pitch, b0 + j, l);
+            gv_load_tq<GK, KB>(wi, g.w + (size_t)stc * g.pitch, b0 + j, l / 4, l % 4);
         } else {
             const uint32_t ncu = (sn / U + NCOL - 1 - gc) / NCOL;  // this thread's unit columns
             const uint32_t ri = k / ncu, uu = gc + NCOL * (k % ncu);
@@ -373,6 +373,137 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvArgs g) {
     }
 }
 
+constexpr uint32_t GQ_T = 512;  // threads of gemv_quad_kernel
+
+// TQ matrices of few strips: four rows (a row quad of a strip) per workgroup.  A workgroup per strip
+// leaves most CUs idle and walks 512 bytes per block alone; here a quad of lanes reads a block's share of
+// its row quad (16 bytes of every 64-byte chunk, the strip's other quads on the same XCD's L2), all of a
+// slice's loads in flight at once, and the chain's terms (m, u, dot, d * sx) are formed in phase 1, so
+// that a chain step is one 16-byte LDS read and two fmas.  Bound by that chain and the staging around it.
+// [320][10240] TQ8_32, us a call at 1 / 2 / 4 rows: 18.3 / 22.9 / 31.8 -> 11.2 / 12.7 / 15.5 (256 threads
+// instead of 512: 11.7 / 14.5 / 19.1).
+template <int GK, int KB, int NA>
+__global__ __launch_bounds__(GQ_T) void gemv_quad_kernel(GemvArgs g) {
+    using T = GvTQ<GK, KB>;
+    constexpr uint32_t S = NA <= 2 ? 256 : 128, NU = S / (GQ_T / 4);  // blocks per slice, units per lane quad
+    constexpr bool XSUM = GK == GK_TQ8;
+    __shared__ __align__(16) int8_t xq[NA][S * KB];
+    __shared__ float2 xs[NA][S];  // sx, u = sx * sum
+    __shared__ int xm[XSUM ? NA : 1][XSUM ? S : 1];
+    __shared__ __align__(16) float4 term[S][NA][4];
+    uint32_t bx = blockIdx.x;
+    xcd_order_1d(gridDim.x, bx);  // a strip's four row quads on one XCD
+    const uint32_t tid = threadIdx.x, row0 = g.r_lo + 4 * bx, rq = row0 / 4 % 4, gi = tid / 4, cl = tid % 4;
+    const uint32_t ca = tid / 4, cr = tid % 4, per = g.pair ? 2u : 1u;  // the chain's (activation, row)
+    const uint8_t* strip = g.w + (size_t)(row0 / 16) * g.pitch;
+    T w[NU];
+    auto load = [&](uint32_t b0, uint32_t sn) {
+#pragma unroll
+        for (uint32_t i = 0; i < NU; i++) {  // past the slice: its last block again
+            const uint32_t j = gi + GQ_T / 4 * i;
+            gv_load_tq<GK, KB>(w[i], strip, b0 + (j < sn ? j : sn - 1), cl, rq);
+        }
+    };
+    for (uint32_t pass = blockIdx.y; pass < g.npass; pass += gridDim.y) {
+        const uint32_t p0 = pass * NA, na = g.m - p0 < NA ? g.m - p0 : NA;
+        float acc = 0.0f;
+        uint32_t sn = g.nb < S ? g.nb : S;
+        load(0, sn);
+        for (uint32_t b0 = 0; b0 < g.nb;) {
+            __syncthreads();  // the previous slice's readers are done
+            const uint32_t pr = sn * KB / 16;
+            for (uint32_t i = tid; i < na * pr; i += GQ_T) {
+                const uint32_t a = i / pr, o = (i % pr) * 16;
+                *reinterpret_cast<int4*>(&xq[a][o]) =
+                    *reinterpret_cast<const int4*>(g.q + (size_t)(p0 + a) * g.k + (size_t)b0 * KB + o);
+            }
+            for (uint32_t i = tid; i < na * sn; i += GQ_T) {
+                const uint32_t a = i / sn, j = i % sn;
+                const size_t bi = (size_t)(p0 + a) * g.nb + b0 + j;
+                const float sx = g.s[bi];
+                xs[a][j] = make_float2(sx, sx * (float)g.su[bi]);  // gemv.rs:143
+                if constexpr (XSUM) {
+                    const int4* xp = reinterpret_cast<const int4*>(g.q + (size_t)(p0 + a) * g.k + (size_t)(b0 + j) * KB);
+                    int v = 0;
+#pragma unroll
+                    for (int t = 0; t < KB / 16; t++) {
+                        const int4 x = xp[t];
+                        v = sdot4(x.w, 0x01010101, sdot4(x.z, 0x01010101, sdot4(x.y, 0x01010101, sdot4(x.x, 0x01010101, v))));
+                    }
+                    xm[a][j] = 128 * v;
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t i = 0; i < NU; i++) {
+                const uint32_t j = gi + GQ_T / 4 * i;
+                if (j >= sn) break;
+                uint32_t lo[T::CPL][4], hi[T::CPL][4];
+                gv_unpack_tq(w[i], rq, lo, hi);
+#pragma unroll
+                for (uint32_t a = 0; a < NA; a++) {
+                    if (a >= na) break;
+                    int dot[4];
+                    gv_dots_tq<GK, KB>(lo, hi, reinterpret_cast<const int*>(&xq[a][j * KB]), cl, dot);
+                    const uint32_t dv[2] = {w[i].d.x, w[i].d.y}, mv[2] = {w[i].m.x, w[i].m.y};
+#pragma unroll
+                    for (int rr = 0; rr < 4; rr++) {
+                        int v = dot[rr];  // over the quad's chunks
+                        v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false);
+                        v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false);
+                        if (cl == 0) {
+                            if constexpr (XSUM) v += xm[a][j];
+                            const float2 x = xs[a][j];
+                            const float d = h2f((uint16_t)(dv[rr / 2] >> (16 * (rr % 2)))), m = h2f((uint16_t)(mv[rr / 2] >> (16 * (rr % 2))));
+                            term[j][a][rr] = make_float4(m, x.y, (float)v, d * x.x);
+                        }
+                    }
+                }
+            }
+            const uint32_t b1 = b0 + sn, sn1 = g.nb - b1 < S ? g.nb - b1 : S;
+            if (b1 < g.nb) load(b1, sn1);
+            __syncthreads();
+            if (ca < na) {  // the chain in block order, eight blocks' terms read while eight are chained
+                auto step = [&](const float4& t) {
+                    acc = __builtin_fmaf(t.x, t.y, acc);
+                    acc = __builtin_fmaf(t.z, t.w, acc);
+                };
+                const uint32_t full = sn / 8 * 8;
+                float4 z0[8], z1[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) z0[i] = term[i][ca][cr];  // unused where full = 0 (in bounds: S >= 8)
+                for (uint32_t j = 0; j < full; j += 16) {
+                    const uint32_t j1 = j + 8 < full ? j + 8 : j, j2 = j + 16 < full ? j + 16 : j;
+#pragma unroll
+                    for (int i = 0; i < 8; i++) z1[i] = term[j1 + i][ca][cr];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) step(z0[i]);
+#pragma unroll
+                    for (int i = 0; i < 8; i++) z0[i] = term[j2 + i][ca][cr];
+                    if (j + 8 < full)
+#pragma unroll
+                        for (int i = 0; i < 8; i++) step(z1[i]);
+                }
+                for (uint32_t j = full; j < sn; j++) step(term[j][ca][cr]);
+            }
+            b0 = b1;
+            sn = sn1;
+        }
+        __syncthreads();
+        float* fin = reinterpret_cast<float*>(&term[0][0][0]);
+        if (ca < na) fin[4 * ca + cr] = acc;
+        __syncthreads();
+        if (tid < 4) {  // the logical rows in order (gemv.rs:150-171)
+            for (uint32_t i = 0; i < na / per; i++) {
+                const float v = g.pair ? fin[8 * i + tid] + fin[8 * i + 4 + tid] : fin[4 * i + tid];
+                const uint32_t lg = p0 / per + i;
+                float* yp = g.y + (size_t)(g.map ? g.map[lg] : lg) * g.ldy + row0 + tid;
+                *yp = g.accumulate ? *yp + v : v;
+            }
+        }
+    }
+}
+
 template <int GK, int KB, int R>
 static hipError_t gemv_go_r(const GemvArgs& g, uint32_t na, dim3 grid, hipStream_t st) {
     if (na <= 1)
@@ -389,6 +520,20 @@ static hipError_t gemv_go_r(const GemvArgs& g, uint32_t na, dim3 grid, hipStream
 template <int GK, int KB>
 static hipError_t gemv_go(const GemvArgs& g, uint32_t na, uint32_t gy, hipStream_t st) {
     const uint32_t n = g.r_hi - g.r_lo;
+    if constexpr (GK >= GK_TQ4) {
+        // up to two such workgroups per CU.  us, strips / row quads at 2 rows: [2048][10240] TQ5_32 (512
+        // workgroups) 23.6 / 15.5, [1024][6400] 16.4 / 9.3; beyond, [12288][2560] 11.3 / 28.5
+        if ((uint64_t)n * gy <= 2048) {
+            const dim3 grid(n / 4, gy);
+            if (na <= 1)
+                gemv_quad_kernel<GK, KB, 1><<<grid, GQ_T, 0, st>>>(g);
+            else if (na <= 2)
+                gemv_quad_kernel<GK, KB, 2><<<grid, GQ_T, 0, st>>>(g);
+            else
+                gemv_quad_kernel<GK, KB, 4><<<grid, GQ_T, 0, st>>>(g);
+            return hipGetLastError();
+        }
+    }
     if (n >= 64 * 1024) return gemv_go_r<GK, KB, 64>(g, na, dim3((n + 63) / 64, gy), st);
     return gemv_go_r<GK, KB, 16>(g, na, dim3((n + 15) / 16, gy), st);
 }

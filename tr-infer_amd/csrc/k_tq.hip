@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256, 4) void tq_layer_kernel(TqArgs g, uint32_t S) 
         const uint32_t n = n_items(sn);
 #pragma unroll
         for (uint32_t i = 0; i < UB; i++)
-            if (k0 + i < n) gv_load_tq<GK, KB>(w[i], sp, b0 + gi + 16 * (k0 + i), l);
+            if (k0 + i < n) gv_load_tq<GK, KB>(w[i], sp, b0 + gi + 16 * (k0 + i), l / 4, l % 4);
     };
     __syncthreads();  // prow / orow
 

@@ -24,11 +24,11 @@ struct GvTQ {
     uint2 d, m;
 };
 
-// The lane's share of TQ block b of the strip at `strip` (lane l of its 16-lane group).
+// The lane's share of TQ block b of the strip at `strip` (chunk lane cl, row quad rq).
 template <int GK, int KB>
-__device__ __forceinline__ void gv_load_tq(GvTQ<GK, KB>& w, const uint8_t* __restrict__ strip, uint32_t b, uint32_t l) {
+__device__ __forceinline__ void gv_load_tq(GvTQ<GK, KB>& w, const uint8_t* __restrict__ strip, uint32_t b, uint32_t cl,
+                                           uint32_t rq) {
     using T = GvTQ<GK, KB>;
-    const uint32_t cl = l / 4, rq = l % 4;
     const uint8_t* blk = strip + (size_t)b * T::BB;
 #pragma unroll
     for (uint32_t t = 0; t < T::CPL; t++) {
@@ -47,17 +47,11 @@ __device__ __forceinline__ void gv_load_tq(GvTQ<GK, KB>& w, const uint8_t* __res
 __device__ __forceinline__ int dpp_ror4_add(int v) { return v + __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, false); }
 __device__ __forceinline__ int dpp_ror8_add(int v) { return v + __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false); }
 
-// The block's 16 row dots against NA staged activation rows: partial dots over the lane's chunks,
-// summed over the group's four chunk lanes (exact integer adds); lane cl = 0 writes its four rows'
-// dots to dl[a][j][r0 + 4 rq + rr] and (d, m) to dm[j][...].
-template <int GK, int KB, int NA, int R, int S>
-__device__ __forceinline__ void gv_terms_tq(const GvTQ<GK, KB>& w, uint32_t l, uint32_t j, uint32_t r0, uint32_t na,
-                                            const int8_t (*xq)[S * KB], const float4 (*xs)[S], float (*dl)[S][R],
-                                            float2 (*dm)[R]) {
+// Its q words unpacked: row 4 rq + rr in chunk t (4/5-bit: low and high nibble planes).
+template <int GK, int KB>
+__device__ __forceinline__ void gv_unpack_tq(const GvTQ<GK, KB>& w, uint32_t rq, uint32_t (&lo)[GvTQ<GK, KB>::CPL][4],
+                                             uint32_t (&hi)[GvTQ<GK, KB>::CPL][4]) {
     using T = GvTQ<GK, KB>;
-    const uint32_t cl = l / 4, rq = l % 4;
-    // q words of row 4 rq + rr in chunk t, unpacked (4/5-bit: low and high nibble planes)
-    uint32_t lo[T::CPL][4], hi[T::CPL][4];
 #pragma unroll
     for (uint32_t t = 0; t < T::CPL; t++) {
         const uint32_t qw[4] = {w.q[t].x, w.q[t].y, w.q[t].z, w.q[t].w};
@@ -78,24 +72,46 @@ __device__ __forceinline__ void gv_terms_tq(const GvTQ<GK, KB>& w, uint32_t l, u
             }
         }
     }
+}
+
+// The four rows' dots of the lane's chunks with the block's activations x (KB bytes).
+template <int GK, int KB>
+__device__ __forceinline__ void gv_dots_tq(const uint32_t (&lo)[GvTQ<GK, KB>::CPL][4], const uint32_t (&hi)[GvTQ<GK, KB>::CPL][4],
+                                           const int* x, uint32_t cl, int (&dot)[4]) {
+    using T = GvTQ<GK, KB>;
+#pragma unroll
+    for (int rr = 0; rr < 4; rr++) dot[rr] = 0;
+#pragma unroll
+    for (uint32_t t = 0; t < T::CPL; t++) {
+        const uint32_t c = cl + 4 * t;
+        if (T::NCH % 4 == 0 || c < T::NCH) {
+            const int xl = x[c];
+            const int xh = T::BITS == 8 ? 0 : x[T::NCH + c];
+#pragma unroll
+            for (int rr = 0; rr < 4; rr++) {
+                dot[rr] = sdot4((int)lo[t][rr], xl, dot[rr]);
+                if constexpr (T::BITS != 8) dot[rr] = sdot4((int)hi[t][rr], xh, dot[rr]);
+            }
+        }
+    }
+}
+
+// The block's 16 row dots against NA staged activation rows: partial dots over the lane's chunks,
+// summed over the group's four chunk lanes (exact integer adds); lane cl = 0 writes its four rows'
+// dots to dl[a][j][r0 + 4 rq + rr] and (d, m) to dm[j][...].
+template <int GK, int KB, int NA, int R, int S>
+__device__ __forceinline__ void gv_terms_tq(const GvTQ<GK, KB>& w, uint32_t l, uint32_t j, uint32_t r0, uint32_t na,
+                                            const int8_t (*xq)[S * KB], const float4 (*xs)[S], float (*dl)[S][R],
+                                            float2 (*dm)[R]) {
+    using T = GvTQ<GK, KB>;
+    const uint32_t cl = l / 4, rq = l % 4;
+    uint32_t lo[T::CPL][4], hi[T::CPL][4];
+    gv_unpack_tq(w, rq, lo, hi);
 #pragma unroll
     for (uint32_t a = 0; a < NA; a++) {
         if (a >= na) break;
-        const int* x = reinterpret_cast<const int*>(&xq[a][j * KB]);
-        int dot[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (uint32_t t = 0; t < T::CPL; t++) {
-            const uint32_t c = cl + 4 * t;
-            if (T::NCH % 4 == 0 || c < T::NCH) {
-                const int xl = x[c];
-                const int xh = T::BITS == 8 ? 0 : x[T::NCH + c];
-#pragma unroll
-                for (int rr = 0; rr < 4; rr++) {
-                    dot[rr] = sdot4((int)lo[t][rr], xl, dot[rr]);
-                    if constexpr (T::BITS != 8) dot[rr] = sdot4((int)hi[t][rr], xh, dot[rr]);
-                }
-            }
-        }
+        int dot[4];
+        gv_dots_tq<GK, KB>(lo, hi, reinterpret_cast<const int*>(&xq[a][j * KB]), cl, dot);
         const int corr = T::BITS == 8 ? 128 * __float_as_int(xs[a][j].z) : 0;
 #pragma unroll
         for (int rr = 0; rr < 4; rr++) {
