@@ -126,6 +126,21 @@ def test_router_mfma_bit_exact(m, E, H):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.abs(got - want).max()
 
 
+@pytest.mark.parametrize("m,E,H", [(159, 96, 768), (160, 33, 768), (161, 512, 1024), (480, 512, 256), (500, 512, 384),
+                                   (193, 70, 192), (290, 16, 2560)])
+def test_router_mfma_chunks_bit_exact(m, E, H):
+    """Either side of the line to the matrix cores (160 rows), every chunk width (256 while each workgroup has
+    a CU, 128, 64; one chunk, odd counts), ragged tiles, and the shared gate's rows beside them."""
+    say(f"router mfma chunks m={m} E={E} H={H}")
+    router = O.gen_normal(2, 1, E * H, 0.02).reshape(E, H)
+    x = O.gen_normal(2, 5, m * H, 1.0).reshape(m, H)
+    shg = O.gen_normal(2, 7, H, 0.02)
+    lg, sh = trmoe.router_logits(to_dev(router), to_dev(x), shexp_gate=to_dev(shg), gemm_order=True)
+    assert np.array_equal(host(lg).view(np.uint32), O.gemm_f32_nt(x, router).view(np.uint32))
+    want = np.array([O.dot(shg, x[i]) for i in range(m)], np.float32)
+    assert np.array_equal(host(sh).view(np.uint32), want.view(np.uint32))
+
+
 def routing_cases(E=512):
     rng = np.random.default_rng(5)
     lg = [rng.standard_normal((8, E)).astype(np.float32),

@@ -172,7 +172,7 @@ __device__ __forceinline__ void router_aux(const float* __restrict__ x, uint32_t
                                            const float* __restrict__ shg, float* __restrict__ sh, const XQuant& xquant,
                                            uint32_t n_dot, uint32_t aux) {
     if (aux < n_dot) {
-        const uint32_t lane = threadIdx.x % WAVE, m0 = (aux * 4 + threadIdx.x / WAVE) * DOT_MR;
+        const uint32_t lane = threadIdx.x % WAVE, m0 = (aux * (blockDim.x / WAVE) + threadIdx.x / WAVE) * DOT_MR;
         if (m0 < m) {
             const uint32_t mr = m - m0 < (uint32_t)DOT_MR ? m - m0 : (uint32_t)DOT_MR;
             float res[DOT_MR];
@@ -309,36 +309,31 @@ __global__ __launch_bounds__(256) void router_gemm_kernel(const float* __restric
         }
 }
 
-// The same gemm_f32_nt order on the matrix cores.  v_mfma_f32_4x4x1f32 is 16 independent 4x4 outer
-// products with accumulate, each element one fma rounded once (the same bits as v_fma_f32): block
-// j of the instruction is chain j of a 4-token x 4-expert tile, its k = 16s + j.  Lane l = 4j + u
-// gives the A value x[token u][k] and the B value w[expert u][k], and gets back acc[token v][expert
-// u] of chain j, v = 0..3.  A wave holds a 16 x 16 tile as 4 x 4 such accumulators (64 VGPRs): per
-// 16-wide step it reads 8 floats from LDS for 16 instructions = 4096 fmas, twice the VALU's fma
-// rate with a quarter of the register tile's LDS reads per fma.  The chains are reduced at the end
-// by the same halving tree (chain j ^ 8, ^ 4, ^ 2, ^ 1: lanes 32, 16, 8, 4 apart).
-// Workgroup tile TM x TE = 32 x 32 (waves 2 x 2), x and router staged in LDS row-major in KC-wide
-// chunks, double-buffered, the global loads two chunks ahead (as in router_gemm_kernel).
-__device__ __forceinline__ float chains_sum(float v) {  // lanes 4j + u, over j: the halving tree
-    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);  // chains j, j ^ 8
-    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(b[0]) + __uint_as_float(b[1]);  // j ^ 4
-    v = v + dpp_f<0x128>(v);                            // row_ror:8: j ^ 2
-    v = v + dpp_f<0x124>(v);                            // row_ror:4: j +- 1, equal after the step before
-    return v;
-}
-template <int KC, int NB>
-__global__ __launch_bounds__(256) void router_mfma_kernel(const float* __restrict__ router,
+// The same gemm_f32_nt order on the matrix cores.  v_mfma_f32_16x16x1f32 is 4 independent 16x16 outer
+// products with accumulate, each element one fma rounded once (the same bits as v_fma_f32, checked on
+// gfx950 over random bit patterns, denormals and infinities).  Lane l = 16 b + r gives block b its
+// A value x[token r][k] and its B value w[expert r][k]; with k = 16 s + 4 b + c the instructions
+// c = 0..3 of step s run the sixteen chains j = 4 b + c of a 16-token x 16-expert tile.  Two waves share
+// a tile, two c each, so a lane's operands of a step are one 8-byte LDS read each of x and w for two
+// instructions (2,048 fmas).  Block b's accumulators come back in registers 4 b + v (token
+// 4 (l / 16) + v, expert l % 16): the halving tree is register adds and one exchange between the waves.
+// Workgroup tile 32 x 32 (eight waves), x and router staged in LDS row-major in KC-wide chunks,
+// double-buffered, the global loads two chunks ahead (as in router_gemm_kernel).
+// Up to about 512 rows the time is a workgroup's walk over its chunks (H = 2048: 0.5 us a chunk beside
+// its MFMAs, hence the wide chunks); at 3,072 the tiles' reads of x and router (0.8 GB through L2).
+// E = 512, H = 2048 x 512 rows 26.5 -> 21.2 us, H = 2560 x 500 rows (VALU tiles before) 40.2 -> 26.3 us
+// against v_mfma_f32_4x4x1f32 tiles (eight 4-byte reads for sixteen instructions).
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+template <int KC>
+__global__ __launch_bounds__(512) void router_mfma_kernel(const float* __restrict__ router,
                                                          const float* __restrict__ bias,
                                                          const float* __restrict__ x, uint32_t m, uint32_t E,
                                                          uint32_t H, float* __restrict__ rlog,
                                                          const float* __restrict__ shg, float* __restrict__ sh,
                                                          XQuant xquant, uint32_t n_dot) {
-    // row pitch 8 mod 32 words: the 4 rows x 8 columns each half-wave reads fall in 32 distinct banks
-    // NB = 4: a wave holds 16 tokens x 16 experts (32 x 32 per workgroup); NB = 2: 16 x 8 (twice
-    // the workgroups for the same rows, where one 32 x 32 tile per CU left a wave per SIMD)
-    constexpr int TM = 32, TE = 8 * NB, XK = KC + 8;
+    // row pitch an odd number of 16-byte pieces
+    constexpr int TM = 32, TE = 32, XK = KC + 4;
     // tiles first, the aux workgroups after them; the tiles in XCD order (xcd_order): an XCD takes
     // a contiguous run of tiles, so the expert tiles of one token tile share its L2's copy of x
     const uint32_t tiles_e = (E + TE - 1) / TE, tiles = tiles_e * ((m + TM - 1) / TM);
@@ -350,58 +345,52 @@ __global__ __launch_bounds__(256) void router_mfma_kernel(const float* __restric
     if (!xcd_order_1d(tiles, bx)) return;
     __shared__ __align__(16) float xs[2][TM][XK];
     __shared__ __align__(16) float wsm[2][TE][XK];
-    const uint32_t tid = threadIdx.x, wv = tid / WAVE, lane = tid % WAVE, j = lane / 4, u = lane % 4;
-    const uint32_t wm = wv / 2, we = wv % 2;  // the wave's 16 x 16 quadrant
+    const uint32_t tid = threadIdx.x, wv = tid / WAVE, lane = tid % WAVE, b = lane / 16, r16 = lane % 16;
+    const uint32_t wm = wv / 2 % 2, we = wv % 2, hf = wv / 4;  // 16 x 16 quadrant, chains c = 2 hf, 2 hf + 1
     const uint32_t m0 = (bx / tiles_e) * TM, e0 = (bx % tiles_e) * TE;
 
     constexpr int XV = TM * KC / 4, WV = TE * KC / 4;  // float4 per chunk
-    constexpr int NV = (XV + WV) / 256;
-    static_assert((XV + WV) % 256 == 0, "every thread stages the same number of float4");
-    float4 sa[NV], sb[NV];
-    auto fetch = [&](uint32_t ck, float4 (&st)[NV]) {
+    constexpr int NV = (XV + WV) / 512;
+    static_assert((XV + WV) % 512 == 0, "every thread stages the same number of float4");
+    v4f sa[NV], sb[NV];
+    auto fetch = [&](uint32_t ck, v4f (&st)[NV]) {
         const uint32_t k0 = ck * KC;
 #pragma unroll
         for (int i = 0; i < NV; i++) {
-            const uint32_t v = tid + 256 * i;
+            const uint32_t v = tid + 512 * i;
             if (v < (uint32_t)XV) {
                 const uint32_t r = v / (KC / 4), c4 = v % (KC / 4);
                 const uint32_t row = m0 + r < m ? m0 + r : m - 1;
-                st[i] = *reinterpret_cast<const float4*>(x + (size_t)row * H + k0 + 4 * c4);
+                st[i] = *reinterpret_cast<const v4f*>(x + (size_t)row * H + k0 + 4 * c4);
             } else {
                 const uint32_t w = v - XV, r = w / (KC / 4), c4 = w % (KC / 4);
                 const uint32_t ex = e0 + r < E ? e0 + r : E - 1;
-                st[i] = *reinterpret_cast<const float4*>(router + (size_t)ex * H + k0 + 4 * c4);
+                st[i] = *reinterpret_cast<const v4f*>(router + (size_t)ex * H + k0 + 4 * c4);
             }
         }
     };
-    auto store = [&](int buf, const float4 (&st)[NV]) {
+    auto store = [&](int buf, const v4f (&st)[NV]) {
 #pragma unroll
         for (int i = 0; i < NV; i++) {
-            const uint32_t v = tid + 256 * i;
+            const uint32_t v = tid + 512 * i;
             float* dst = v < (uint32_t)XV ? &xs[buf][v / (KC / 4)][4 * (v % (KC / 4))]
                                           : &wsm[buf][(v - XV) / (KC / 4)][4 * ((v - XV) % (KC / 4))];
-            reinterpret_cast<float2*>(dst)[0] = make_float2(st[i].x, st[i].y);
-            reinterpret_cast<float2*>(dst)[1] = make_float2(st[i].z, st[i].w);
+            *reinterpret_cast<v4f*>(dst) = st[i];
         }
     };
-    v4f acc[4][NB];
+    v16f acc[2];  // [c - 2 hf][4 b + v]
 #pragma unroll
-    for (int a = 0; a < 4; a++)
+    for (int c = 0; c < 2; c++)
 #pragma unroll
-        for (int b = 0; b < NB; b++) acc[a][b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < 16; i++) acc[c][i] = 0.0f;
     auto compute = [&](int buf) {
+        const float* xr = &xs[buf][16 * wm + r16][4 * b + 2 * hf];
+        const float* wr = &wsm[buf][16 * we + r16][4 * b + 2 * hf];
 #pragma unroll
         for (int s = 0; s < KC / 16; s++) {
-            const uint32_t c = 16 * s + j;
-            float xv[4], wvv[NB];
+            const v2f xv = *reinterpret_cast<const v2f*>(xr + 16 * s), wvv = *reinterpret_cast<const v2f*>(wr + 16 * s);
 #pragma unroll
-            for (int a = 0; a < 4; a++) xv[a] = xs[buf][16 * wm + 4 * a + u][c];
-#pragma unroll
-            for (int b = 0; b < NB; b++) wvv[b] = wsm[buf][4 * NB * we + 4 * b + u][c];
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int b = 0; b < NB; b++) acc[a][b] = rank1(xv[a], wvv[b], acc[a][b]);
+            for (int c = 0; c < 2; c++) acc[c] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[c], wvv[c], acc[c], 0, 0, 0);
         }
     };
     const uint32_t nchunk = H / KC;
@@ -420,27 +409,27 @@ __global__ __launch_bounds__(256) void router_mfma_kernel(const float* __restric
         compute(1);
         __syncthreads();
     }
-    // every lane ends with all 4 NB (a, b) sums; lane (j, u), j < 4 NB, stores tile (a, b) =
-    // (j / NB, j % NB): tokens 4a + v, expert 4b + u
-    float outv[4];
+    // the halving tree over chains j = 4 b + c: j ^ 8 and j ^ 4 are b's bits, j ^ 2 the other wave's
+    // chains (through LDS), j ^ 1 c's low bit
+    float t[2][4];
 #pragma unroll
-    for (int v = 0; v < 4; v++) outv[v] = 0.0f;
+    for (int c = 0; c < 2; c++)
 #pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < NB; b++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const float t = chains_sum(acc[a][b][v]);
-                outv[v] = j == (uint32_t)(NB * a + b) ? t : outv[v];
-            }
-    const uint32_t ex = e0 + 4 * NB * we + 4 * (j % NB) + u;
-    if (j < 4 * NB && ex < E) {
+        for (int v = 0; v < 4; v++) t[c][v] = (acc[c][v] + acc[c][8 + v]) + (acc[c][4 + v] + acc[c][12 + v]);
+    float* ex2 = &xs[0][0][0] + (wv % 4 * 64 + lane) * 8;  // 8 KB, past the last chunk's barrier
+    if (hf) {
+        *reinterpret_cast<v4f*>(ex2) = v4f{t[0][0], t[0][1], t[0][2], t[0][3]};
+        *reinterpret_cast<v4f*>(ex2 + 4) = v4f{t[1][0], t[1][1], t[1][2], t[1][3]};
+    }
+    __syncthreads();
+    const uint32_t ex = e0 + 16 * we + r16;
+    if (!hf && ex < E) {
         const float bb = bias ? bias[ex] : 0.0f;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            const uint32_t row = m0 + 16 * wm + 4 * (j / NB) + v;
-            if (row < m) rlog[(size_t)row * E + ex] = bias ? outv[v] + bb : outv[v];
+            const float sum = (t[0][v] + ex2[v]) + (t[1][v] + ex2[4 + v]);
+            const uint32_t row = m0 + 16 * wm + 4 * b + v;
+            if (row < m) rlog[(size_t)row * E + ex] = bias ? sum + bb : sum;
         }
     }
 }
@@ -453,7 +442,7 @@ struct GemmCfg {
 };
 // (a chunk must divide H: the kernel walks H / KC whole chunks; 64- and 16-wide chunks take the
 // K-split slices of a tiled router, e.g. 2560 / 8 = 320 columns)
-static const GemmCfg kGemmCfg[] = {{256, 128, 1}, {64, 256, 5}, {0, 512, 2}, {0, 128, 3}, {0, 64, 6}, {0, 16, 7}};
+static const GemmCfg kGemmCfg[] = {{64, 256, 5}, {0, 512, 2}, {0, 128, 3}, {0, 64, 6}, {0, 16, 7}};
 
 template <int RM, int RE, int QM, int KC, bool DB>
 static void launch_gemm_cfg(const float* router, const float* bias, const float* x, uint32_t m, uint32_t E,
@@ -494,23 +483,25 @@ hipError_t launch_router_logits(const float* router, const float* bias, const fl
         const uint32_t n_dot = shexp_gate ? (chunks + 3) / 4 : 0u;
         const uint32_t n_aux = n_dot + (xquant ? (m * (H / 32) * 4 + 255) / 256 : 0u);
         const XQuant& xq = xquant ? *xquant : none;
-        // the matrix-core gemm from 512 rows (config 4: 160 -> 91 us; M = 512: 35 -> 31 us, its 256
-        // workgroups one per CU).  64-wide chunks: 32 and 128 were no faster, nor chunks stored
-        // transposed so that a lane reads its four steps as one float4
-        if (m >= 512 && H % 64 == 0 && m < 1024) {  // 16 x 8 per wave: two waves per SIMD at M = 512
-            const uint32_t tiles = ((E + 15) / 16) * ((m + 31) / 32);
-            router_mfma_kernel<64, 2><<<tiles + n_aux, 256, 0, st>>>(router, bias, x, m, E, H, rlog, shexp_gate, sh, xq,
-                                                                    n_dot);
-            return hipGetLastError();
-        } else if (m >= 512 && H % 64 == 0) {
-            const uint32_t tiles = ((E + 31) / 32) * ((m + 31) / 32);
-            router_mfma_kernel<64, 4><<<tiles + n_aux, 256, 0, st>>>(router, bias, x, m, E, H, rlog, shexp_gate, sh, xq,
-                                                                  n_dot);
+        // the matrix-core gemm from 160 rows.  us, VALU tiles / matrix cores, E = 512: H = 2048 x 128 rows
+        // 15.2 / 17.9, x 200 25.5 / 18.4, x 384 26.4 / 18.7, x 500 33 / 21.4; H = 2560 x 128 17.4 / 21.7, x
+        // 200 31 / 22.3, x 500 40 / 26.3.  256-wide chunks (133 KB of LDS) while every workgroup has a CU
+        // of its own, else 128 (two per CU): x 384 18.7 / 21.4, x 500 25.9 / 21.4, x 3072 109 / 87
+        if (m >= 160 && H % 64 == 0) {
+            const uint32_t tiles = ((E + 31) / 32) * ((m + 31) / 32), nd = shexp_gate ? (chunks + 7) / 8 : 0u;
+            const uint32_t grid = tiles + nd + (xquant ? (m * (H / 32) * 4 + 511) / 512 : 0u);
+#define MFMA_GO(KC) router_mfma_kernel<KC><<<grid, 512, 0, st>>>(router, bias, x, m, E, H, rlog, shexp_gate, sh, xq, nd)
+            if (H % 256 == 0 && grid <= 256)
+                MFMA_GO(256);
+            else if (H % 128 == 0)
+                MFMA_GO(128);
+            else
+                MFMA_GO(64);
+#undef MFMA_GO
             return hipGetLastError();
         }
         switch (id) {
 #define GEMM_ARGS router, bias, x, m, E, H, rlog, shexp_gate, sh, xq, n_dot, n_aux, st
-            case 1: launch_gemm_cfg<4, 4, 4, 128, true>(GEMM_ARGS); break;
             case 2: launch_gemm_cfg<1, 2, 16, 512, false>(GEMM_ARGS); break;
             case 5: launch_gemm_cfg<4, 2, 4, 256, true>(GEMM_ARGS); break;
             case 6: launch_gemm_cfg<1, 2, 16, 64, true>(GEMM_ARGS); break;
