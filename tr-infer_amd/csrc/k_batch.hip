@@ -45,8 +45,8 @@ __device__ __forceinline__ uint32_t load_ids(const Workspace& ws, uint32_t t, ui
 // the wave totals).  kc4 = ceil(largest selection / 4).
 constexpr uint32_t DT = DISPATCH_WAVES * 64;  // tokens per round
 // split: leave the scatter to scatter_kernel (many workgroups) and store the per-(64-token chunk,
-// expert) first positions in ws.doff instead: pass 1 stores each chunk's counts there, and one
-// prefix per expert over the chunks turns them into positions (no second pass over the tokens).
+// expert) first positions in ws.doff instead: from each chunk's counts (count_kernel's over several
+// rounds, one round's own masks) one prefix per expert over the chunks (no second pass over the tokens).
 __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace ws, uint32_t m, uint32_t kc4,
                                                                        int split) {
     const uint32_t E = ws.E, tid = threadIdx.x;
@@ -84,19 +84,31 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
         __syncthreads();
     };
 
-    // pass 1: per-expert counts
-    for (uint32_t e = tid; e < E; e += DT) cnt[e] = 0;
-    for (uint32_t r = 0; r < rounds; r++) {
+    // pass 1: per-expert counts (over several rounds count_kernel left them per chunk in ws.doff)
+    if (split && rounds > 1) {
+        for (uint32_t e = tid; e < E; e += DT) {
+            uint32_t c = 0;
+            for (uint32_t ch0 = 0; ch0 < nchunks; ch0 += 16) {  // 16 counts requested at once
+                uint32_t v[16];
+#pragma unroll
+                for (int j = 0; j < 16; j++) {
+                    const uint32_t ch = ch0 + j < nchunks ? ch0 + j : nchunks - 1;
+                    v[j] = ws.doff[(size_t)ch * E + e];
+                }
+#pragma unroll
+                for (int j = 0; j < 16; j++) c += ch0 + j < nchunks ? v[j] : 0u;
+            }
+            cnt[e] = c;
+        }
+    } else {
+        for (uint32_t e = tid; e < E; e += DT) cnt[e] = 0;
+    }
+    for (uint32_t r = 0; r < (split && rounds > 1 ? 0u : rounds); r++) {
         load_tok(r);
         build_masks();
         for (uint32_t e = tid; e < E; e += DT) {
             uint32_t c = cnt[e];
-            for (uint32_t w = 0; w < DISPATCH_WAVES; w++) {
-                const uint32_t pc = popc64(masks[w * E + e]);
-                const uint32_t ch = r * DISPATCH_WAVES + w;  // 64-token chunk
-                if (split && rounds > 1 && ch < nchunks) ws.doff[(size_t)ch * E + e] = pc;  // its count, for now
-                c += pc;
-            }
+            for (uint32_t w = 0; w < DISPATCH_WAVES; w++) c += popc64(masks[w * E + e]);
             cnt[e] = c;
         }
         if (rounds > 1) __syncthreads();
@@ -233,6 +245,26 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
             }
         if (rounds > 1) __syncthreads();
     }
+}
+
+// The entries of every expert in one 64-token chunk (a workgroup per chunk), into ws.doff.
+__global__ __launch_bounds__(256) void count_kernel(Workspace ws, uint32_t m, uint32_t kc4) {
+    extern __shared__ uint32_t ccnt[];  // [E]
+    const uint32_t E = ws.E, tid = threadIdx.x, t = blockIdx.x * 64 + tid / 4;
+    for (uint32_t e = tid; e < E; e += 256) ccnt[e] = 0u;
+    __syncthreads();
+    if (t < m) {
+        const uint32_t n = ws.n_sel[t];
+        for (uint32_t q = tid % 4; q < kc4; q += 4) {
+            const uint4 v = reinterpret_cast<const uint4*>(ws.ids + (size_t)t * K_MAX)[q];
+            const uint32_t id[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++)
+                if (4 * q + i < n) atomicAdd(&ccnt[id[i]], 1u);
+        }
+    }
+    __syncthreads();
+    for (uint32_t e = tid; e < E; e += 256) ws.doff[(size_t)blockIdx.x * E + e] = ccnt[e];
 }
 
 // The scatter of a split dispatch: one wave per 64-token chunk, the same lane-mask ranks.
@@ -413,6 +445,9 @@ hipError_t launch_dispatch(const Workspace& ws, uint32_t m, uint32_t kcap, hipSt
     // from a few hundred tokens on, one workgroup's scattered stores dominate: spread them
     const int split = geo::dispatch_split(m) ? 1 : 0;
     if (split && geo::doff_elems(m, ws.E) > geo::doff_elems(ws.m_max, ws.E)) return hipErrorInvalidValue;
+    // over several rounds of DT tokens the counts come from a workgroup per chunk: one workgroup building
+    // every round's masks took 30 of 41 us at 3,072 tokens (41 -> 5 + 12 us); one round keeps its masks
+    if (split && m > DT) count_kernel<<<geo::chunks(m), 256, E * 4, st>>>(ws, m, (kcap + 3) / 4);
     dispatch_kernel<<<1, DT, lds, st>>>(ws, m, (kcap + 3) / 4, split);
     if (split) scatter_kernel<<<geo::chunks(m), 64, E * 12, st>>>(ws, m, (kcap + 3) / 4);
     return hipGetLastError();
