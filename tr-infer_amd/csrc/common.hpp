@@ -282,6 +282,15 @@ __device__ __forceinline__ T row16_allreduce(T v, Op op) {
     v = op(v, mv(v, std::integral_constant<int, 0x140>{}));  // row_mirror
     return v;
 }
+// The same over each half-wave of 32 lanes: the two rows of 16 meet in a permlane16 swap (registers; an
+// xor shuffle is an LDS round trip per step).
+template <typename T, typename Op>
+__device__ __forceinline__ T row32_allreduce(T v, Op op) {
+    v = row16_allreduce(v, op);
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return op(__builtin_bit_cast(T, (uint32_t)p[0]), __builtin_bit_cast(T, (uint32_t)p[1]));
+}
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) { return wave_reduce_u32<false>(v); }
 
 // Token (activation row) of entry row `row` of a grouped work item; rows past the item reuse its

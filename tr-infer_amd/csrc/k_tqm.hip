@@ -1273,7 +1273,7 @@ struct HcArgs {
 
 // batch: silu(lo * (1 / hc)) of every row quantised per 32, once, into the operand image.  A
 // thread per value and a half-wave per block (lr % 32 == 0: a block is 32 consecutive values of
-// one row): the lanes reduce the block's |max| and sums with xor shuffles (max and integer sums:
+// one row): the lanes reduce the block's |max| and sums in registers (row32_allreduce; max and integer sums:
 // any order gives quant_block_regs' values for finite input), stage their q bytes in LDS, and
 // four lanes write the block's 8-byte operand pieces.
 __global__ __launch_bounds__(256) void hc_quant_kernel(const float* __restrict__ lo, uint32_t m, uint32_t lr,
@@ -1288,19 +1288,13 @@ __global__ __launch_bounds__(256) void hc_quant_kernel(const float* __restrict__
         const float y = lo[j] * inv;
         x = j % lr < body ? silu512(y) : y * sigmoid_libm(y);
     }
-    float amax = __builtin_fabsf(x);
-#pragma unroll
-    for (int o = 16; o >= 1; o /= 2) amax = mx_ps(amax, __shfl_xor(amax, o, 32));
+    const float amax = row32_allreduce(__builtin_fabsf(x), [](float a, float b) { return mx_ps(a, b); });
     const float sc = amax / 127.0f;
     const float qinv = amax > 0.0f ? 127.0f / amax : 0.0f;
     const int32_t qi = cvt_rne(x * qinv);
     const int8_t qb = sat_i8(qi);
-    int sum = qi, bs = qb;
-#pragma unroll
-    for (int o = 16; o >= 1; o /= 2) {
-        sum += __shfl_xor(sum, o, 32);
-        bs += __shfl_xor(bs, o, 32);
-    }
+    auto add = [](int a, int b) { return a + b; };
+    const int sum = row32_allreduce((int)qi, add), bs = row32_allreduce((int)qb, add);
     qs[hb][k] = qb;
     __syncthreads();
     if (!live || k >= 6) return;
@@ -1377,7 +1371,8 @@ __global__ __launch_bounds__(512) void hc_mix_kernel(HcArgs g) {
     if constexpr (DEC) {
         // the one row's silu(lo / hc) and its per-32 quantisation (two levels with hiprec), a
         // value per lane: block b = j / 32 of value j = tid + nthr c is a half-wave, whose lanes
-        // reduce the block's |max| and sums with xor shuffles (max and integer sums: any order
+        // reduce the block's |max| and sums in registers (row32_allreduce, thirty xor shuffles before, each
+        // an LDS round trip in a chain: 8.1 -> 6.8 us at the real shape; max and integer sums: any order
         // gives quant_block_regs' values for finite input) and write their q bytes in the 16-row
         // tile image, level lv as A row lv
         long* As = reinterpret_cast<long*>(smem);
@@ -1408,19 +1403,13 @@ __global__ __launch_bounds__(512) void hc_mix_kernel(HcArgs g) {
                 const float y = lv[c] / (float)g.hc;
                 float x = y * sigmoid_libm(y);
                 for (uint32_t lev = 0; lev < P; lev++) {
-                    float amax = __builtin_fabsf(x);
-#pragma unroll
-                    for (int o = 16; o >= 1; o /= 2) amax = mx_ps(amax, __shfl_xor(amax, o, 32));
+                    const float amax = row32_allreduce(__builtin_fabsf(x), [](float a, float b) { return mx_ps(a, b); });
                     const float sc = amax / 127.0f;
                     const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
                     const int32_t qi = cvt_rne(x * inv);
                     const int8_t qb = sat_i8(qi);
-                    int sum = qi, bs = qb;
-#pragma unroll
-                    for (int o = 16; o >= 1; o /= 2) {
-                        sum += __shfl_xor(sum, o, 32);
-                        bs += __shfl_xor(bs, o, 32);
-                    }
+                    auto add = [](int a, int b) { return a + b; };
+                    const int sum = row32_allreduce((int)qi, add), bs = U8 ? row32_allreduce((int)qb, add) : 0;
                     Ab[((b * 4 + k / 8) * 16 + lev) * 8 + k % 8] = qb;
                     if (k == 0) {
                         SU[b * 16 + lev] = make_float2(sc, sc * (float)sum);
