@@ -10,6 +10,9 @@
 // loads are in flight during a slice.
 // [12288][2560] TQ5_32 x 512 rows: 983 us as GEMV passes of 4 rows (each decoding the weights
 // again) -> 82 us.  Of these about 60 are the tiles (without the staging) and 40 the staging alone.
+// The staging counts its load instructions: row pairs' d and m and the whole plane chunk as wide loads
+// instead of 2-byte ones took [12288][2560] TQ4_32 x 16 / 512 from 30 / 75 to 25 / 72 us and [24000][2560]
+// TQ8_32 x 512 from 190 to 170.
 #include "tq.hpp"
 
 namespace trk {
@@ -47,11 +50,11 @@ struct GmW {
     static constexpr uint32_t PW = GM_ROWS * 16 + 16;  // bytes per piece, padded off the banks' period
     using T = GvTQ<GK_TQ4 <= GK ? GK : GK_TQ4, KB>;
     // TQ: a unit is 16 bytes of a block's q chunk (4 rows x 4 values, two nibbles each at 4/5 bits)
-    static constexpr uint32_t UPB = T::NCH * 4, NU = TQ ? 8 * NBLK * UPB / 256 : 0, ND = GM_ROWS * NBLK / 256;
+    static constexpr uint32_t UPB = T::NCH * 4, NU = TQ ? 8 * NBLK * UPB / 256 : 0, ND = GM_ROWS / 2 * NBLK / 256;
     static constexpr uint32_t NW = GK == GK_Q4K ? 3 : GK == GK_Q6K ? 3 : GK == GK_Q51 ? 3 : 4;
     u4v v[TQ ? NU : NW];
-    uint32_t pl[GK == GK_TQ5 ? NU : 1];                    // the 5-bit plane's two 16-bit pieces
-    uint32_t hd[TQ ? ND : 4];            // TQ: (d, m) halves; GGUF: the rest
+    u4v pl[GK == GK_TQ5 ? NU : 1];   // the 5-bit plane's chunk
+    uint32_t hd[TQ ? 2 * ND : 4];    // TQ: row pairs' d and m; GGUF: the rest
 
     __device__ __forceinline__ void load(const GemmArgs& g, uint32_t row0, uint32_t b0, uint32_t nblk) {
         const uint32_t tid = threadIdx.x;
@@ -63,19 +66,15 @@ struct GmW {
                 const uint8_t* blk = g.w + (size_t)(st < ns ? st : ns - 1) * g.pitch +
                                      (size_t)(b0 + (j < nblk ? j : nblk - 1)) * T::BB;
                 v[i] = *reinterpret_cast<const u4v*>(blk + 64 + 16 * e);
-                if constexpr (GK == GK_TQ5) {
-                    const uint8_t* p = blk + 64 + 64 * T::NCH + 16 * (e / 4) + 2 * (e % 4);
-                    pl[i] = (uint32_t)*reinterpret_cast<const uint16_t*>(p) |
-                            (uint32_t)*reinterpret_cast<const uint16_t*>(p + 8) << 16;
-                }
+                if constexpr (GK == GK_TQ5) pl[i] = *reinterpret_cast<const u4v*>(blk + 64 + 64 * T::NCH + 16 * (e / 4));
             }
 #pragma unroll
             for (uint32_t i = 0; i < ND; i++) {
-                const uint32_t u = tid + 256 * i, r = u % 16, j = u / 16 % NBLK, st = s0 + u / 16 / NBLK;
+                const uint32_t u = tid + 256 * i, r2 = u % 8, j = u / 8 % NBLK, st = s0 + u / 8 / NBLK;
                 const uint8_t* blk = g.w + (size_t)(st < ns ? st : ns - 1) * g.pitch +
                                      (size_t)(b0 + (j < nblk ? j : nblk - 1)) * T::BB;
-                hd[i] = (uint32_t)reinterpret_cast<const uint16_t*>(blk)[r] |
-                        (uint32_t)reinterpret_cast<const uint16_t*>(blk)[16 + r] << 16;
+                hd[2 * i] = reinterpret_cast<const uint32_t*>(blk)[r2];
+                hd[2 * i + 1] = reinterpret_cast<const uint32_t*>(blk)[8 + r2];
             }
         } else {  // a thread per (row, 64 of the slice's 128 values); k is a multiple of 256
             const uint32_t r = row0 + tid / 2, c = tid % 2, sl = b0 / NBLK;
@@ -114,7 +113,12 @@ struct GmW {
 #pragma unroll
             for (uint32_t i = 0; i < NU; i++) {
                 const uint32_t u = tid + 256 * i, e = u % UPB, j = u / UPB % NBLK, st = u / UPB / NBLK;
-                const uint32_t c = e / 4, row = 16 * st + 4 * (e % 4);
+                const uint32_t c = e / 4, rq = e % 4, row = 16 * st + 4 * rq;
+                uint32_t ql = 0, qh = 0;  // the fifth bits of the four rows' low and high halves
+                if constexpr (GK == GK_TQ5) {
+                    ql = (rq < 2 ? pl[i].x : pl[i].y) >> (16 * (rq % 2));
+                    qh = (rq < 2 ? pl[i].z : pl[i].w) >> (16 * (rq % 2));
+                }
                 // words c (low nibbles) and NCH + c (high) of the block's KB / 4; 8 bits: word c
                 const uint32_t lo = KB / 4 * j + c, hi = lo + T::NCH;
                 uint32_t* pl0 = reinterpret_cast<uint32_t*>(wb + lo / 4 * PW + row * 16) + lo % 4;
@@ -127,8 +131,8 @@ struct GmW {
                     } else {
                         uint32_t a = w & 0x0f0f0f0fu, b = (w >> 4) & 0x0f0f0f0fu;
                         if constexpr (GK == GK_TQ5) {
-                            a |= q5_hi4((pl[i] >> (4 * rr)) & 0xfu);
-                            b |= q5_hi4((pl[i] >> (16 + 4 * rr)) & 0xfu);
+                            a |= q5_hi4((ql >> (4 * rr)) & 0xfu);
+                            b |= q5_hi4((qh >> (4 * rr)) & 0xfu);
                         }
                         pl0[4 * rr] = a;
                         ph0[4 * rr] = b;
@@ -137,8 +141,10 @@ struct GmW {
             }
 #pragma unroll
             for (uint32_t i = 0; i < ND; i++) {
-                const uint32_t u = tid + 256 * i, r = u % 16, j = u / 16 % NBLK, st = u / 16 / NBLK;
-                dm[j][16 * st + r] = make_float2(h2f((uint16_t)(hd[i] & 0xffffu)), h2f((uint16_t)(hd[i] >> 16)));
+                const uint32_t u = tid + 256 * i, r2 = u % 8, j = u / 8 % NBLK, st = u / 8 / NBLK;
+                const uint32_t d = hd[2 * i], m = hd[2 * i + 1];
+                *reinterpret_cast<float4*>(&dm[j][16 * st + 2 * r2]) =
+                    make_float4(h2f((uint16_t)(d & 0xffffu)), h2f((uint16_t)(m & 0xffffu)), h2f((uint16_t)(d >> 16)), h2f((uint16_t)(m >> 16)));
             }
         } else {
             const uint32_t r = tid / 2, c = tid % 2, n = b0 / NBLK % 2;
@@ -224,7 +230,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(GemmArgs g) {
     __shared__ __align__(16) uint8_t wb[8 * SL * W::PW];
     __shared__ __align__(16) float xsc[NBLK][2][TOK];  // sx, u = sx * sum in rank1's lane order
     __shared__ __align__(16) int xsum[XSUM ? NBLK : 1][XSUM ? TOK : 4];
-    __shared__ float2 dm[NBLK][GM_ROWS];
+    __shared__ __align__(16) float2 dm[NBLK][GM_ROWS];
     const uint32_t tid = threadIdx.x, lane = tid % 64, wv = tid / 64, h = lane / 32, c32 = lane % 32;
     uint32_t idx = 0;
     if (!xcd_order_1d(gridDim.x, idx)) return;
@@ -361,7 +367,7 @@ static hipError_t gemm_go(GemmArgs g, hipStream_t st) {
     const uint32_t rb = (g.r_hi - g.r_lo + GM_ROWS - 1) / GM_ROWS, t32 = (g.m + 31) / 32, t64 = (g.m + 63) / 64;
     // 32 activation rows a workgroup (a tile per wave, 256-value slices) while three such workgroups
     // fit every CU, 64 (two tiles per wave, the unpacked weights serving both, 128-value slices)
-    // beyond.  us at 32 / 64 rows: [12288][2560] TQ5_32 x 128 41 / 53, x 256 52 / 65, x 512 93 / 82;
+    // beyond.  us at 32 / 64 rows: [12288][2560] TQ5_32 x 128 40 / 53, x 256 53 / 65, x 512 93 / 82;
     // [24576][2048] Q4_K x 128 42 / 50, x 256 74 / 65, x 512 134 / 115
     if ((uint64_t)rb * t32 <= 3 * 256) {
         g.tb = t32;

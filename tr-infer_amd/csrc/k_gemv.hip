@@ -543,7 +543,7 @@ hipError_t launch_gemv(const Mat& w, uint32_t item, uint32_t s0, uint32_t s1, ui
                        const uint32_t* rows, int accumulate, hipStream_t st) {
     // Many activation rows run as MFMA tiles once the GEMV would need seven workgroups per CU (a
     // workgroup per strip and pass of four rows): below that its shorter K walk wins.  us, GEMV / tiles:
-    // [12288][2560] TQ4_32 x 8 (6 per CU) 22 / 31, x 16 (12) 35 / 31; [2560][640] TQ5_16 x 32 (5) 13 /
+    // [12288][2560] TQ4_32 x 8 (6 per CU) 22 / 25, x 16 (12) 35 / 25; [2560][640] TQ5_16 x 32 (5) 13 /
     // 14; [4096][4096] Q6_K x 16 (4) 47 / 80, x 32 (8) 90 / 81; [24576][2048] Q4_K x 8 (12) 48 / 26
     // A row map may repeat rows in an order of its own and stays here.
     if (!rows && m > GV_NA && (uint64_t)(s1 - s0) * ((m + GV_NA - 1) / GV_NA) >= 7 * 256)
