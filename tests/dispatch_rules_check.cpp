@@ -1,0 +1,38 @@
+// CPU-only check of the dispatch rules (tr-infer_amd/csrc/geometry.hpp) at sizes where both forms were
+// timed on an MI355X: the rule takes the faster one.  Built with g++ by tests/test_geometry.py; the
+// argument names the rule.  Prints "ok" and the number of cases, or the first failing one and exits 1.
+#include <cstdio>
+#include <cstring>
+
+#include "geometry.hpp"
+
+using namespace trk::geo;
+
+static int n = 0, bad = 0;
+static void expect(bool got, bool want, const char* what, unsigned a, unsigned b, unsigned c) {
+    n++;
+    if (got == want) return;
+    bad++;
+    std::printf("FAIL %s (%u, %u, %u): %d\n", what, a, b, c, (int)got);
+}
+
+// (m, E, H): few experts leave the matrix-core tiles without workgroups, whatever the rows
+static void router() {
+    const unsigned valu[][3] = {{160, 16, 2048}, {200, 64, 2048}, {200, 128, 2560}, {300, 128, 2048}, {400, 128, 2048},
+                                {200, 256, 2048}, {176, 256, 1024}, {160, 384, 2048}, {500, 64, 2048}, {1023, 32, 2048},
+                                {800, 16, 2560}, {300, 16, 256}, {500, 64, 320}, {200, 128, 192}, {200, 128, 640},
+                                {159, 512, 2048}, {500, 512, 2000}};
+    const unsigned mfma[][3] = {{160, 512, 2048}, {176, 384, 2048}, {300, 256, 2048}, {500, 128, 2048}, {500, 256, 2560},
+                                {500, 512, 2560}, {512, 512, 2048}, {1500, 16, 2048}, {3072, 512, 2048}, {300, 128, 320},
+                                {300, 256, 192}, {800, 64, 640}};
+    for (auto& c : valu) expect(router_on_mfma(c[0], c[1], c[2]), false, "router_on_mfma", c[0], c[1], c[2]);
+    for (auto& c : mfma) expect(router_on_mfma(c[0], c[1], c[2]), true, "router_on_mfma", c[0], c[1], c[2]);
+}
+
+int main(int argc, char** argv) {
+    const char* what = argc > 1 ? argv[1] : "";
+    if (!std::strcmp(what, "router")) router();
+    if (!n || bad) return 1;
+    std::printf("ok %d\n", n);
+    return 0;
+}

@@ -114,7 +114,7 @@ def test_router_gemm_tiles_bit_exact(m):
 @pytest.mark.parametrize("m,E,H", [(512, 512, 2048), (700, 96, 768), (1024, 512, 2048), (1100, 80, 512),
                                    (1057, 96, 2560), (3072, 512, 2048)])
 def test_router_mfma_bit_exact(m, E, H):
-    """The matrix-core router gemm (m >= 512): the same bits as gemm_f32_nt's chains and halving
+    """The matrix-core router gemm: the same bits as gemm_f32_nt's chains and halving
     tree, with ragged token and expert tiles, a bias, and the full shapes of configs 3 and 4."""
     say(f"router mfma m={m} E={E} H={H}")
     router = O.gen_normal(2, 1, E * H, 0.02).reshape(E, H)
@@ -127,10 +127,12 @@ def test_router_mfma_bit_exact(m, E, H):
 
 
 @pytest.mark.parametrize("m,E,H", [(159, 96, 768), (160, 33, 768), (161, 512, 1024), (480, 512, 256), (500, 512, 384),
-                                   (193, 70, 192), (290, 16, 2560)])
+                                   (193, 70, 192), (290, 16, 2560), (330, 161, 192), (1025, 40, 64), (1025, 33, 768),
+                                   (401, 257, 512), (400, 120, 768), (400, 121, 768), (1024, 61, 320), (401, 33, 256)])
 def test_router_mfma_chunks_bit_exact(m, E, H):
-    """Either side of the line to the matrix cores (160 rows), every chunk width (256 while each workgroup has
-    a CU, 128, 64; one chunk, odd counts), ragged tiles, and the shared gate's rows beside them."""
+    """Either side of the line to the matrix cores (160 rows, and enough experts to fill the VALU tiles'
+    workgroups: 480 of them up to 400 rows), every chunk width (256 while each workgroup has a CU, 128, 64; one
+    chunk, odd counts), ragged tiles, and the shared gate's rows beside them."""
     say(f"router mfma chunks m={m} E={E} H={H}")
     router = O.gen_normal(2, 1, E * H, 0.02).reshape(E, H)
     x = O.gen_normal(2, 5, m * H, 1.0).reshape(m, H)

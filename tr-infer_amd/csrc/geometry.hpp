@@ -85,6 +85,30 @@ inline uint32_t decode_down_wgs(uint32_t H) { return H / DN_R; }
 inline uint32_t tq_gateup_tiles(uint32_t F) { return 2 * F / 16; }
 inline uint32_t tq_down_tiles(uint32_t H) { return H / 16; }
 
+// Router logits in gemm order (k_router.hip) from 64 rows: VALU tiles of 16 rows x 8 experts (x 2 where
+// H is no multiple of 256), or matrix-core tiles of 32 x 32.
+inline uint64_t router_valu_wgs(uint32_t m, uint32_t E, uint32_t H) {
+    const uint64_t te = H % 256 == 0 ? 8 : 2;
+    return (E + te - 1) / te * ((m + 15) / 16);
+}
+// A matrix-core tile takes as long however few they are (the walk of one workgroup: 16 us at H = 2048),
+// while the VALU tiles' time goes with their workgroups per CU.  us, VALU / matrix cores, the kernel alone
+// and in a layer (x quantised beside it), H = 2048:
+//   up to a workgroup per CU: E = 64 x 200 rows 11.6 / 16.0 and 12.6 / 16.1, E = 16 x 800 11.7 / 16.0
+//   and 15 / 18, E = 64 x 500 13.2 / 16.0 and 15.2 / 18.2;
+//   up to two, from a few hundred rows on beside as many quantising workgroups: E = 128 x 400 (400 of
+//   them) 14.3 / 15.9 and 16.9 / 17.8, E = 384 x 160 (480) 14.3 / 16.0 and 15.0 / 16.0, but E = 128 x 500
+//   (512) 15.4 / 16.0 and 19.5 / 18.0, E = 256 x 256 (512) 14.6 / 16.0 and 18.5 / 16.8;
+//   beyond: E = 512 x 160 (640) 18.2 / 15.9, x 300 27.7 / 18.5.
+// H = 640, 320 and 192 (K-split slices): E = 64 x 500 (1024) 7.3 / 7.6, 5.1 / 5.8 and 4.1 / 4.7, E = 128 x
+// 300 (1216) 9.6 / 7.6, 6.9 / 5.9 and 5.3 / 4.7.
+inline bool router_on_mfma(uint32_t m, uint32_t E, uint32_t H) {
+    if (m < 160 || H % 64) return false;
+    const uint64_t valu = router_valu_wgs(m, E, H);
+    if (H % 256) return valu > 1024;
+    return valu > (m <= 400 ? 480u : m <= 1024 ? 256u : 0u);
+}
+
 // Every invariant a call of m rows with kcap selections per token relies on; returns nullptr when
 // they hold, else what failed.  tq: the experts are TQ strips (k_tq.hip), not GGUF superblocks.
 inline const char* check_call(const Caps& c, uint32_t m, uint32_t kcap, bool tq = false) {

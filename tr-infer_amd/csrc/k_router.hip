@@ -322,7 +322,8 @@ __global__ __launch_bounds__(256) void router_gemm_kernel(const float* __restric
 // Up to about 512 rows the time is a workgroup's walk over its chunks (H = 2048: 0.5 us a chunk beside
 // its MFMAs, hence the wide chunks); at 3,072 the tiles' reads of x and router (0.8 GB through L2).
 // E = 512, H = 2048 x 512 rows 26.5 -> 21.2 us, H = 2560 x 500 rows (VALU tiles before) 40.2 -> 26.3 us
-// against v_mfma_f32_4x4x1f32 tiles (eight 4-byte reads for sixteen instructions).
+// against v_mfma_f32_4x4x1f32 tiles (eight 4-byte reads for sixteen instructions).  Where it runs:
+// geo::router_on_mfma.
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 template <int KC>
@@ -483,11 +484,9 @@ hipError_t launch_router_logits(const float* router, const float* bias, const fl
         const uint32_t n_dot = shexp_gate ? (chunks + 3) / 4 : 0u;
         const uint32_t n_aux = n_dot + (xquant ? (m * (H / 32) * 4 + 255) / 256 : 0u);
         const XQuant& xq = xquant ? *xquant : none;
-        // the matrix-core gemm from 160 rows.  us, VALU tiles / matrix cores, E = 512: H = 2048 x 128 rows
-        // 15.2 / 17.9, x 200 25.5 / 18.4, x 384 26.4 / 18.7, x 500 33 / 21.4; H = 2560 x 128 17.4 / 21.7, x
-        // 200 31 / 22.3, x 500 40 / 26.3.  256-wide chunks (133 KB of LDS) while every workgroup has a CU
-        // of its own, else 128 (two per CU): x 384 18.7 / 21.4, x 500 25.9 / 21.4, x 3072 109 / 87
-        if (m >= 160 && H % 64 == 0) {
+        // 256-wide chunks (133 KB of LDS) while every workgroup has a CU of its own, else 128 (two per CU): E =
+        // 512, H = 2048 x 384 rows 18.7 / 21.4 us, x 500 25.9 / 21.4, x 3072 109 / 87
+        if (geo::router_on_mfma(m, E, H)) {
             const uint32_t tiles = ((E + 31) / 32) * ((m + 31) / 32), nd = shexp_gate ? (chunks + 7) / 8 : 0u;
             const uint32_t grid = tiles + nd + (xquant ? (m * (H / 32) * 4 + 511) / 512 : 0u);
 #define MFMA_GO(KC) router_mfma_kernel<KC><<<grid, 512, 0, st>>>(router, bias, x, m, E, H, rlog, shexp_gate, sh, xq, nd)
