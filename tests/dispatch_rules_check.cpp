@@ -29,9 +29,18 @@ static void router() {
     for (auto& c : mfma) expect(router_on_mfma(c[0], c[1], c[2]), true, "router_on_mfma", c[0], c[1], c[2]);
 }
 
+// (tiles, quantising workgroups beside them): 256-wide chunks where both find CUs
+static void chunks() {
+    const unsigned wide[][2] = {{256, 0}, {160, 1}, {208, 1}, {224, 1}, {1, 1}};
+    const unsigned narrow[][2] = {{257, 0}, {256, 1}, {240, 1}, {320, 0}};
+    for (auto& c : wide) expect(router_wide_chunks(c[0], c[1] != 0), true, "router_wide_chunks", c[0], c[1], 0);
+    for (auto& c : narrow) expect(router_wide_chunks(c[0], c[1] != 0), false, "router_wide_chunks", c[0], c[1], 0);
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "router")) router();
+    if (!std::strcmp(what, "chunks")) chunks();
     if (!n || bad) return 1;
     std::printf("ok %d\n", n);
     return 0;

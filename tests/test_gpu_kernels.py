@@ -131,8 +131,8 @@ def test_router_mfma_bit_exact(m, E, H):
                                    (401, 257, 512), (400, 120, 768), (400, 121, 768), (1024, 61, 320), (401, 33, 256)])
 def test_router_mfma_chunks_bit_exact(m, E, H):
     """Either side of the line to the matrix cores (160 rows, and enough experts to fill the VALU tiles'
-    workgroups: 480 of them up to 400 rows), every chunk width (256 while each workgroup has a CU, 128, 64; one
-    chunk, odd counts), ragged tiles, and the shared gate's rows beside them."""
+    workgroups: 480 of them up to 400 rows), every chunk width (256 while the tiles and the shared
+    gate's workgroups have CUs of their own, 128, 64; one chunk, odd counts), ragged tiles, and the shared gate's rows beside them."""
     say(f"router mfma chunks m={m} E={E} H={H}")
     router = O.gen_normal(2, 1, E * H, 0.02).reshape(E, H)
     x = O.gen_normal(2, 5, m * H, 1.0).reshape(m, H)

@@ -109,6 +109,13 @@ inline bool router_on_mfma(uint32_t m, uint32_t E, uint32_t H) {
     return valu > (m <= 400 ? 480u : m <= 1024 ? 256u : 0u);
 }
 
+// The matrix-core tiles walk 256-wide chunks (133 KB of LDS: a CU each) while they and what runs beside them
+// have CUs of their own, else 128-wide ones (two tiles per CU).  In a layer the quantising workgroups carry
+// the tiles' LDS too, in a few turns on the CUs that the tiles leave: an eighth of the GPU is enough, none
+// is not.  us in a layer, 256 / 128 wide: E = 512, H = 2048 x 300 rows (160 tiles) 19.1 / 21.9, x 400
+// (208) 18.9 / 22.1, x 500 (256) 26.4 / 21.9; the tiles alone x 500 18.9 / 21.9, x 640 (320) 33.7 / 29.2.
+inline bool router_wide_chunks(uint64_t tiles, bool aux) { return tiles + (aux ? 32 : 0) <= 256; }
+
 // Every invariant a call of m rows with kcap selections per token relies on; returns nullptr when
 // they hold, else what failed.  tq: the experts are TQ strips (k_tq.hip), not GGUF superblocks.
 inline const char* check_call(const Caps& c, uint32_t m, uint32_t kcap, bool tq = false) {

@@ -484,13 +484,11 @@ hipError_t launch_router_logits(const float* router, const float* bias, const fl
         const uint32_t n_dot = shexp_gate ? (chunks + 3) / 4 : 0u;
         const uint32_t n_aux = n_dot + (xquant ? (m * (H / 32) * 4 + 255) / 256 : 0u);
         const XQuant& xq = xquant ? *xquant : none;
-        // 256-wide chunks (133 KB of LDS) while every workgroup has a CU of its own, else 128 (two per CU): E =
-        // 512, H = 2048 x 384 rows 18.7 / 21.4 us, x 500 25.9 / 21.4, x 3072 109 / 87
         if (geo::router_on_mfma(m, E, H)) {
             const uint32_t tiles = ((E + 31) / 32) * ((m + 31) / 32), nd = shexp_gate ? (chunks + 7) / 8 : 0u;
             const uint32_t grid = tiles + nd + (xquant ? (m * (H / 32) * 4 + 511) / 512 : 0u);
 #define MFMA_GO(KC) router_mfma_kernel<KC><<<grid, 512, 0, st>>>(router, bias, x, m, E, H, rlog, shexp_gate, sh, xq, nd)
-            if (H % 256 == 0 && grid <= 256)
+            if (H % 256 == 0 && geo::router_wide_chunks(tiles, grid > tiles))
                 MFMA_GO(256);
             else if (H % 128 == 0)
                 MFMA_GO(128);
