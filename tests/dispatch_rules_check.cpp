@@ -3,6 +3,7 @@
 // argument names the rule.  Prints "ok" and the number of cases, or the first failing one and exits 1.
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 
 #include "geometry.hpp"
 
@@ -37,10 +38,23 @@ static void chunks() {
     for (auto& c : narrow) expect(router_wide_chunks(c[0], c[1] != 0), false, "router_wide_chunks", c[0], c[1], 0);
 }
 
+// n workgroups of t threads as rows of a grid: none lost, under 2^32 threads a row
+static void grids() {
+    const unsigned long long ns[] = {1, 255, 256, 8388600, 8388607, 8388608, 8392609, 16777216, 100000000};
+    for (unsigned t : {256u, 512u})
+        for (unsigned long long v : ns) {
+            const Grid2 g = grid_run(v, t);
+            expect((unsigned long long)g.x * t <= 0xffffffffull && (unsigned long long)g.x * g.y >= v &&
+                           (g.y == 1 ? g.x == v : g.x % 8 == 0 && (unsigned long long)g.x * (g.y - 1) < v),
+                   true, "grid_run", (unsigned)v, t, g.x);
+        }
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "router")) router();
     if (!std::strcmp(what, "chunks")) chunks();
+    if (!std::strcmp(what, "grids")) grids();
     if (!n || bad) return 1;
     std::printf("ok %d\n", n);
     return 0;

@@ -143,6 +143,23 @@ def test_router_mfma_chunks_bit_exact(m, E, H):
     assert np.array_equal(host(sh).view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("n,H", [(32 * 2897, 64), (23200, 16)])
+def test_router_more_tiles_than_one_grid_row(n, H):
+    """n x n logits whose tiles pass 2^32 threads (32 x 32 of 512 threads, 34 GB; 16 x 2 of 256): every sampled
+    row, the last ones too, as a call of its own gives it."""
+    torch = torch_dev()
+    say(f"router {n} x {n} logits, H={H}")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    x, router = (torch.randn((n, H), device="cuda", generator=gen) for _ in range(2))
+    lg, _ = trmoe.router_logits(router, x, gemm_order=True)
+    for r in (0, 31, n // 2, n - 40, n - 1):
+        one, _ = trmoe.router_logits(router, x[r:r + 1].contiguous(), gemm_order=True)
+        assert torch.equal(lg[r].view(torch.int32), one[0].view(torch.int32)), r
+    del lg
+    torch.cuda.empty_cache()
+
+
 def routing_cases(E=512):
     rng = np.random.default_rng(5)
     lg = [rng.standard_normal((8, E)).astype(np.float32),

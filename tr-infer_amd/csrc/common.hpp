@@ -312,9 +312,10 @@ __device__ __forceinline__ bool xcd_order(uint32_t n_items, uint32_t& col, uint3
     return true;
 }
 
+// The workgroup's place in a run of them over x and y (geo::grid_run).
+__device__ __forceinline__ uint32_t run_id() { return blockIdx.x + gridDim.x * blockIdx.y; }
 // The same for a 1-D grid whose first n workgroups are live: id -> its place in XCD order.
-__device__ __forceinline__ bool xcd_order_1d(uint32_t n, uint32_t& idx) {
-    const uint32_t id = blockIdx.x;
+__device__ __forceinline__ bool xcd_order_1d(uint32_t n, uint32_t& idx, uint32_t id) {
     if (id >= n) return false;
     const uint32_t x = id % 8, slot = id / 8, base = n / 8, rem = n % 8;
     idx = x * base + (x < rem ? x : rem) + slot;

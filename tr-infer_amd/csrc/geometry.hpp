@@ -85,6 +85,17 @@ inline uint32_t decode_down_wgs(uint32_t H) { return H / DN_R; }
 inline uint32_t tq_gateup_tiles(uint32_t F) { return 2 * F / 16; }
 inline uint32_t tq_down_tiles(uint32_t H) { return H / 16; }
 
+// A launch's workgroups over x and y: a launch holds less than 2^32 threads in x, and a kernel that numbers its
+// workgroups in one run takes the rest as rows of y (x * y >= n; multiples of 8 in x keep id % 8 the XCD).
+struct Grid2 {
+    uint32_t x, y;
+};
+inline Grid2 grid_run(uint64_t n, uint32_t threads) {
+    const uint64_t most = 0xffffffffull / threads / 8 * 8;
+    if (n <= most) return Grid2{(uint32_t)n, 1};
+    return Grid2{(uint32_t)most, (uint32_t)((n + most - 1) / most)};
+}
+
 // Router logits in gemm order (k_router.hip) from 64 rows: VALU tiles of 16 rows x 8 experts (x 2 where
 // H is no multiple of 256), or matrix-core tiles of 32 x 32.
 inline uint64_t router_valu_wgs(uint32_t m, uint32_t E, uint32_t H) {

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(GemmArgs g) {
     __shared__ __align__(16) float2 dm[NBLK][GM_ROWS];
     const uint32_t tid = threadIdx.x, lane = tid % 64, wv = tid / 64, h = lane / 32, c32 = lane % 32;
     uint32_t idx = 0;
-    if (!xcd_order_1d(gridDim.x, idx)) return;
+    if (!xcd_order_1d(gridDim.x, idx, blockIdx.x)) return;
     const uint32_t t0 = idx % g.tb * TOK, row0 = g.r_lo + idx / g.tb * GM_ROWS;
     const uint32_t wr = wv % WR * (RT * 32), wt = wv / WR * 32;
 

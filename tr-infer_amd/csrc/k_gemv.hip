@@ -392,7 +392,7 @@ __global__ __launch_bounds__(GQ_T) void gemv_quad_kernel(GemvArgs g) {
     __shared__ int xm[XSUM ? NA : 1][XSUM ? S : 1];
     __shared__ __align__(16) float4 term[S][NA][4];
     uint32_t bx = blockIdx.x;
-    xcd_order_1d(gridDim.x, bx);  // a strip's four row quads on one XCD
+    xcd_order_1d(gridDim.x, bx, blockIdx.x);  // a strip's four row quads on one XCD
     const uint32_t tid = threadIdx.x, row0 = g.r_lo + 4 * bx, rq = row0 / 4 % 4, gi = tid / 4, cl = tid % 4;
     const uint32_t ca = tid / 4, cr = tid % 4, per = g.pair ? 2u : 1u;  // the chain's (activation, row)
     const uint8_t* strip = g.w + (size_t)(row0 / 16) * g.pitch;

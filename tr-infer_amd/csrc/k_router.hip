@@ -192,8 +192,9 @@ __global__ __launch_bounds__(256) void router_gemm_kernel(const float* __restric
                                                          const float* __restrict__ shg, float* __restrict__ sh,
                                                          XQuant xquant, uint32_t n_dot, uint32_t n_aux) {
     constexpr int QE = 16 / QM, TM = QM * RM, TE = QE * RE;
-    if (blockIdx.x < n_aux) {  // workgroup-uniform
-        router_aux(x, m, H, shg, sh, xquant, n_dot, blockIdx.x);
+    const uint32_t id = run_id();
+    if (id < n_aux) {  // workgroup-uniform
+        router_aux(x, m, H, shg, sh, xquant, n_dot, id);
         return;
     }
     // rows between the 16-lane groups of one wave (q = 0..3): x rows differ when qm does
@@ -204,8 +205,9 @@ __global__ __launch_bounds__(256) void router_gemm_kernel(const float* __restric
     __shared__ __align__(16) float xs[NB][TM][XK];
     __shared__ __align__(16) float wsm[NB][TE][WK];
     const uint32_t tid = threadIdx.x, j = tid % 16, q = tid / 16, qm = q / QE, qe = q % QE;
-    const uint32_t tiles_e = (E + TE - 1) / TE, bx = blockIdx.x - n_aux;
+    const uint32_t tiles_e = (E + TE - 1) / TE, bx = id - n_aux;
     const uint32_t m0 = (bx / tiles_e) * TM, e0 = (bx % tiles_e) * TE;
+    if (m0 >= m) return;  // past the last tile (workgroup-uniform)
 
     // staging: TM rows of x and TE rows of the router, KC columns each, as float4 along k
     constexpr int XV = TM * KC / 4, WV = TE * KC / 4;  // float4 per chunk
@@ -332,18 +334,19 @@ __global__ __launch_bounds__(512) void router_mfma_kernel(const float* __restric
                                                          const float* __restrict__ x, uint32_t m, uint32_t E,
                                                          uint32_t H, float* __restrict__ rlog,
                                                          const float* __restrict__ shg, float* __restrict__ sh,
-                                                         XQuant xquant, uint32_t n_dot) {
+                                                         XQuant xquant, uint32_t n_dot, uint32_t n_run) {
     // row pitch an odd number of 16-byte pieces
     constexpr int TM = 32, TE = 32, XK = KC + 4;
     // tiles first, the aux workgroups after them; the tiles in XCD order (xcd_order): an XCD takes
     // a contiguous run of tiles, so the expert tiles of one token tile share its L2's copy of x
     const uint32_t tiles_e = (E + TE - 1) / TE, tiles = tiles_e * ((m + TM - 1) / TM);
-    if (blockIdx.x >= tiles) {  // workgroup-uniform
-        router_aux(x, m, H, shg, sh, xquant, n_dot, blockIdx.x - tiles);
+    const uint32_t id = run_id();
+    if (id >= tiles) {  // workgroup-uniform
+        if (id < n_run) router_aux(x, m, H, shg, sh, xquant, n_dot, id - tiles);
         return;
     }
     uint32_t bx;
-    if (!xcd_order_1d(tiles, bx)) return;
+    if (!xcd_order_1d(tiles, bx, id)) return;
     __shared__ __align__(16) float xs[2][TM][XK];
     __shared__ __align__(16) float wsm[2][TE][XK];
     const uint32_t tid = threadIdx.x, wv = tid / WAVE, lane = tid % WAVE, b = lane / 16, r16 = lane % 16;
@@ -451,8 +454,9 @@ static void launch_gemm_cfg(const float* router, const float* bias, const float*
                             uint32_t n_dot, uint32_t n_aux, hipStream_t st) {
     constexpr uint32_t TM = QM * RM, TE = (16 / QM) * RE;
     const uint32_t tiles = ((E + TE - 1) / TE) * ((m + TM - 1) / TM);
-    router_gemm_kernel<RM, RE, QM, KC, DB><<<n_aux + tiles, 256, 0, st>>>(router, bias, x, m, E, H, rlog, shg, sh, xq,
-                                                                         n_dot, n_aux);
+    const geo::Grid2 gr = geo::grid_run((uint64_t)n_aux + tiles, 256);
+    router_gemm_kernel<RM, RE, QM, KC, DB><<<dim3(gr.x, gr.y), 256, 0, st>>>(router, bias, x, m, E, H, rlog, shg, sh, xq,
+                                                                            n_dot, n_aux);
 }
 
 hipError_t launch_router_logits(const float* router, const float* bias, const float* shexp_gate, const float* x,
@@ -487,7 +491,9 @@ hipError_t launch_router_logits(const float* router, const float* bias, const fl
         if (geo::router_on_mfma(m, E, H)) {
             const uint32_t tiles = ((E + 31) / 32) * ((m + 31) / 32), nd = shexp_gate ? (chunks + 7) / 8 : 0u;
             const uint32_t grid = tiles + nd + (xquant ? (m * (H / 32) * 4 + 511) / 512 : 0u);
-#define MFMA_GO(KC) router_mfma_kernel<KC><<<grid, 512, 0, st>>>(router, bias, x, m, E, H, rlog, shexp_gate, sh, xq, nd)
+            const geo::Grid2 gr = geo::grid_run(grid, 512);
+#define MFMA_GO(KC) \
+    router_mfma_kernel<KC><<<dim3(gr.x, gr.y), 512, 0, st>>>(router, bias, x, m, E, H, rlog, shexp_gate, sh, xq, nd, grid)
             if (H % 256 == 0 && geo::router_wide_chunks(tiles, grid > tiles))
                 MFMA_GO(256);
             else if (H % 128 == 0)
