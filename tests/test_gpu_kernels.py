@@ -349,6 +349,26 @@ def test_gemv_many_rows_bit_exact(fmt, kb, rows, K, pair, m, strips):
         assert np.array_equal(got[:, :c0], base[:, :c0]) and np.array_equal(got[:, c1:], base[:, c1:]), acc
 
 
+def test_gemv_more_tiles_than_one_grid_row():
+    """A strip against so many activation rows that its tiles of 256 threads pass 2^32 threads: every sampled
+    row, the last ones too, as a call of its own gives it."""
+    torch = torch_dev()
+    m, kb = (1 << 30) + 200, 16
+    if torch.cuda.mem_get_info()[0] < 120 << 30:
+        pytest.skip("needs 100 GB of free memory")
+    say(f"gemv of {m} activation rows")
+    tq = to_dev(random_tq(3, 16, kb, 4, kb))
+    q = torch.arange(m, dtype=torch.int32, device="cuda").view(m, 1).expand(m, kb // 4).contiguous().view(torch.int8)
+    s = torch.full((m, 1), 0.5, device="cuda")
+    su = torch.full((m, 1), 3, dtype=torch.int32, device="cuda")
+    y = trmoe.gemv(tq, 16, kb, trmoe.FMT_TQ4_16, 0, 1, kb, q, s, su)
+    for r in (0, 63, m // 2, m - 300, m - 1):
+        one = trmoe.gemv(tq, 16, kb, trmoe.FMT_TQ4_16, 0, 1, kb, q[r:r + 1].clone(), s[:1], su[:1])
+        assert torch.equal(y[r].view(torch.int32), one[0].view(torch.int32)), r
+    del y, q, s, su
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("m", [1, 70, 300, 512])
 def test_designed_rounding_orders(m):
     """The designed cases that pin the oracle's f32 orders (test_oracle.py: test_gemv_epilogue_order,

@@ -34,7 +34,7 @@ struct GemmArgs {
     const float* s;       // [m][nb]
     const int32_t* su;    // [m][nb]
     uint32_t m;           // physical activation rows
-    uint32_t tb;          // blocks of TOK activation rows
+    uint32_t tb, n;       // blocks of TOK activation rows; tiles
     int pair;
     float* y;
     uint32_t ldy;
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(GemmArgs g) {
     __shared__ __align__(16) float2 dm[NBLK][GM_ROWS];
     const uint32_t tid = threadIdx.x, lane = tid % 64, wv = tid / 64, h = lane / 32, c32 = lane % 32;
     uint32_t idx = 0;
-    if (!xcd_order_1d(gridDim.x, idx, blockIdx.x)) return;
+    if (!xcd_order_1d(g.n, idx, run_id())) return;
     const uint32_t t0 = idx % g.tb * TOK, row0 = g.r_lo + idx / g.tb * GM_ROWS;
     const uint32_t wr = wv % WR * (RT * 32), wt = wv / WR * 32;
 
@@ -371,10 +371,13 @@ static hipError_t gemm_go(GemmArgs g, hipStream_t st) {
     // [24576][2048] Q4_K x 128 42 / 50, x 256 74 / 65, x 512 134 / 115
     if ((uint64_t)rb * t32 <= 3 * 256) {
         g.tb = t32;
-        gemm_rows_kernel<GK, KB, 4, 2><<<rb * t32, 256, 0, st>>>(g);
+        g.n = rb * t32;
+        gemm_rows_kernel<GK, KB, 4, 2><<<g.n, 256, 0, st>>>(g);
     } else {
         g.tb = t64;
-        gemm_rows_kernel<GK, KB, 2, 1><<<rb * t64, 256, 0, st>>>(g);
+        g.n = rb * t64;
+        const geo::Grid2 gr = geo::grid_run(g.n, 256);
+        gemm_rows_kernel<GK, KB, 2, 1><<<dim3(gr.x, gr.y), 256, 0, st>>>(g);
     }
     return hipGetLastError();
 }
@@ -392,7 +395,7 @@ hipError_t launch_gemm(const Mat& w, uint32_t item, uint32_t s0, uint32_t s1, ui
     g.s = s;
     g.su = su;
     g.m = m;
-    g.tb = 0;
+    g.tb = g.n = 0;
     g.pair = pair;
     g.y = y;
     g.ldy = ldy;
