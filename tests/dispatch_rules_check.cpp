@@ -50,11 +50,22 @@ static void grids() {
         }
 }
 
+// (blocks of 128 weight rows, of 32 activation rows): the 32-row form up to three workgroups per CU and where
+// the 64-row one would run empty halves
+static void gemm() {
+    const unsigned narrow[][3] = {{96, 1, 32}, {96, 8, 32}, {192, 4, 32}, {768, 1, 32}, {782, 1, 32}, {1172, 1, 16},
+                                  {1940, 1, 32}, {192, 5, 32}, {192, 5, 16}, {32, 24, 16}, {1024, 3, 32}};
+    const unsigned wide[][3] = {{96, 16, 32}, {192, 8, 32}, {192, 8, 16}, {768, 2, 32}, {1940, 2, 16}, {16, 64, 32}, {1024, 3, 16}};
+    for (auto& c : narrow) expect(gemm_narrow(c[0], c[1], c[2]), true, "gemm_narrow", c[0], c[1], c[2]);
+    for (auto& c : wide) expect(gemm_narrow(c[0], c[1], c[2]), false, "gemm_narrow", c[0], c[1], c[2]);
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "router")) router();
     if (!std::strcmp(what, "chunks")) chunks();
     if (!std::strcmp(what, "grids")) grids();
+    if (!std::strcmp(what, "gemm")) gemm();
     if (!n || bad) return 1;
     std::printf("ok %d\n", n);
     return 0;

@@ -311,7 +311,7 @@ def test_gemv_few_rows_bit_exact(bits, kb, rows, K, pair, m, strips):
 
 # Enough (strip, pass) workgroups for the MFMA tiles: every codec, ragged row and activation tiles (the
 # last workgroup nearly empty), k short of a slice and past one, strip sub-ranges, pairs, accumulate;
-# 64-row workgroups from 769 of 32 rows (m = 520 at 48 row blocks)
+# 64-row workgroups past three of 32 rows per CU (m = 520 at 48 row blocks)
 GEMM_CASES = [(O.FMT_Q4_K, 32, 1000, 512, False, 129, None), (O.FMT_Q4_K, 16, 440, 256, True, 145, (1, 27)),
               (O.FMT_Q6_K, 16, 520, 768, False, 241, (3, 33)), (O.FMT_Q8_0, 32, 1160, 256, False, 100, None),
               (O.FMT_Q8_0, 16, 240, 512, True, 260, None), (O.FMT_Q5_1, 32, 480, 256, False, 241, None),
@@ -319,7 +319,10 @@ GEMM_CASES = [(O.FMT_Q4_K, 32, 1000, 512, False, 129, None), (O.FMT_Q4_K, 16, 44
               ((4, 16), 16, 1800, 80, False, 65, None), ((5, 32), 32, 700, 320, True, 91, (2, 44)),
               ((5, 16), 16, 2560, 176, False, 45, (0, 157)), ((8, 32), 32, 28700, 32, False, 5, None),
               ((8, 16), 16, 400, 640, False, 289, None), ((8, 32), 32, 6100, 160, False, 520, None),
-              ((5, 16), 16, 6100, 272, True, 260, None), (O.FMT_Q6_K, 16, 6100, 256, False, 520, None)]
+              ((5, 16), 16, 6100, 272, True, 260, None), (O.FMT_Q6_K, 16, 6100, 256, False, 520, None),
+              # past three workgroups per CU: one block of activation rows, a half-empty one, three blocks
+              ((4, 32), 32, 98400, 32, False, 5, None), ((8, 32), 32, 98400, 32, False, 33, None),
+              ((5, 32), 32, 33000, 64, False, 90, None)]
 
 
 @pytest.mark.parametrize("fmt,kb,rows,K,pair,m,strips", GEMM_CASES)

@@ -127,6 +127,20 @@ inline bool router_on_mfma(uint32_t m, uint32_t E, uint32_t H) {
 // (208) 18.9 / 22.1, x 500 (256) 26.4 / 21.9; the tiles alone x 500 18.9 / 21.9, x 640 (320) 33.7 / 29.2.
 inline bool router_wide_chunks(uint64_t tiles, bool aux) { return tiles + (aux ? 32 : 0) <= 256; }
 
+// trk_gemv tiles (k_gemm.hip) of 128 weight rows (rb blocks of them) x 32 activation rows (t32 blocks) or x 64.
+// A 64-row workgroup serves two tiles from one unpacking and takes half as long again as a 32-row one (a
+// third at kb 16); up to three per CU the 32-row form is ahead however they divide, beyond it where the
+// 64-row form has empty halves.  us, 32 / 64 rows a workgroup:
+//   2 and 1 per CU: [12288][2560] TQ5_32 x 128 rows 40 / 53; 3 and 2: x 256 53 / 65, [4096][4096] TQ5_16 x 768
+//   147 / 154 and Q6_K 167 / 166 (kb 16: two resident, the third a second round, as dear as the 64-row form);
+//   6 and 3: [12288][2560] TQ5_32 x 512 93 / 82, [24576][2048] Q4_K x 256 79 / 63, TQ5_16 x 256 137 / 105;
+//   4 and 3: [24576][2048] Q4_K x 160 55 / 60, TQ5_16 x 160 95 / 103; 12 and 8: [131072][768] Q6_K x 96 125 / 112;
+//   one block: [150016][2048] Q4_K x 8 (5 and 5) 62 / 93, [248320][2560] TQ8_32 x 8 (8 and 8) 162 / 233.
+inline bool gemm_narrow(uint64_t rb, uint64_t t32, uint32_t kb) {
+    const uint64_t c32 = (rb * t32 + 255) / 256, c64 = (rb * ((t32 + 1) / 2) + 255) / 256;
+    return c32 <= 3 || (kb == 16 ? 3 * c32 <= 4 * c64 : 2 * c32 <= 3 * c64);
+}
+
 // Every invariant a call of m rows with kcap selections per token relies on; returns nullptr when
 // they hold, else what failed.  tq: the experts are TQ strips (k_tq.hip), not GGUF superblocks.
 inline const char* check_call(const Caps& c, uint32_t m, uint32_t kcap, bool tq = false) {

@@ -216,8 +216,9 @@ struct GmW {
 };
 
 // WR x (4 / WR) waves over 128 weight rows x TOK activation rows (a wave: 4 / WR tiles of 32 weight
-// rows at 32 activation rows), slices of SL x 128 values.  Each tile is three resident workgroups'
-// worth of registers; a wave's per-block cost is its VALU and rank1 issue (about 48 VALU
+// rows at 32 activation rows), slices of SL x 128 values.  Three workgroups per CU are resident at kb 32 and
+// in the 64-row form at kb 16, two in the 32-row form at kb 16 (62 to 64 KB of LDS) and in the 64-row form of
+// 8-bit TQ (186 and 195 registers); a wave's per-block cost is its VALU and rank1 issue (about 48 VALU
 // instructions, an int8 MFMA and four rank1 a tile), not the LDS reads (prefetching them: no change).
 template <int GK, int KB, int WR, int SL>
 __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(GemmArgs g) {
@@ -365,20 +366,16 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(GemmArgs g) {
 template <int GK, int KB>
 static hipError_t gemm_go(GemmArgs g, hipStream_t st) {
     const uint32_t rb = (g.r_hi - g.r_lo + GM_ROWS - 1) / GM_ROWS, t32 = (g.m + 31) / 32, t64 = (g.m + 63) / 64;
-    // 32 activation rows a workgroup (a tile per wave, 256-value slices) while three such workgroups
-    // fit every CU, 64 (two tiles per wave, the unpacked weights serving both, 128-value slices)
-    // beyond.  us at 32 / 64 rows: [12288][2560] TQ5_32 x 128 40 / 53, x 256 53 / 65, x 512 93 / 82;
-    // [24576][2048] Q4_K x 128 42 / 50, x 256 74 / 65, x 512 134 / 115
-    if ((uint64_t)rb * t32 <= 3 * 256) {
-        g.tb = t32;
-        g.n = rb * t32;
-        gemm_rows_kernel<GK, KB, 4, 2><<<g.n, 256, 0, st>>>(g);
-    } else {
-        g.tb = t64;
-        g.n = rb * t64;
-        const geo::Grid2 gr = geo::grid_run(g.n, 256);
+    // 32 activation rows a workgroup (a tile per wave, 256-value slices) or 64 (two tiles per wave, the
+    // unpacked weights serving both, 128-value slices): geo::gemm_narrow
+    const bool narrow = geo::gemm_narrow(rb, t32, KB);
+    g.tb = narrow ? t32 : t64;
+    g.n = rb * g.tb;
+    const geo::Grid2 gr = geo::grid_run(g.n, 256);
+    if (narrow)
+        gemm_rows_kernel<GK, KB, 4, 2><<<dim3(gr.x, gr.y), 256, 0, st>>>(g);
+    else
         gemm_rows_kernel<GK, KB, 2, 1><<<dim3(gr.x, gr.y), 256, 0, st>>>(g);
-    }
     return hipGetLastError();
 }
 
