@@ -60,12 +60,26 @@ static void gemm() {
     for (auto& c : wide) expect(gemm_narrow(c[0], c[1], c[2]), false, "gemm_narrow", c[0], c[1], c[2]);
 }
 
+// (GEMV workgroups, TQ codec or 0, k): the tiles from the GEMV's third round of 1024, before it on GGUF formats
+// and short columns
+static void tiles() {
+    const unsigned gemv[][3] = {{1791, 0, 4096}, {1791, 0x410, 80}, {1792, 0x420, 3072}, {1792, 0x420, 1536}, {1792, 0x520, 1024},
+                                {2048, 0x520, 2560}, {1920, 0x520, 2560}, {2048, 0x820, 4096}, {1800, 0x820, 10240},
+                                {1792, 0x810, 768}, {1920, 0x420, 10240}, {2060, 0x820, 10240}};
+    const unsigned mfma[][3] = {{1792, 0, 256}, {1792, 0, 10240}, {1792, 0x420, 1024}, {1792, 0x510, 768}, {1792, 0x810, 512},
+                                {1792, 0x820, 768}, {2048, 0x420, 3072}, {2064, 0x520, 2560}, {2064, 0x820, 2048},
+                                {2320, 0x820, 10240}, {2080, 0x420, 10240}, {98304, 0x520, 2560}};
+    for (auto& c : gemv) expect(gemv_tiles(c[0], c[1], c[2]), false, "gemv_tiles", c[0], c[1], c[2]);
+    for (auto& c : mfma) expect(gemv_tiles(c[0], c[1], c[2]), true, "gemv_tiles", c[0], c[1], c[2]);
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "router")) router();
     if (!std::strcmp(what, "chunks")) chunks();
     if (!std::strcmp(what, "grids")) grids();
     if (!std::strcmp(what, "gemm")) gemm();
+    if (!std::strcmp(what, "tiles")) tiles();
     if (!n || bad) return 1;
     std::printf("ok %d\n", n);
     return 0;

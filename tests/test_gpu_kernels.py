@@ -322,7 +322,10 @@ GEMM_CASES = [(O.FMT_Q4_K, 32, 1000, 512, False, 129, None), (O.FMT_Q4_K, 16, 44
               ((5, 16), 16, 6100, 272, True, 260, None), (O.FMT_Q6_K, 16, 6100, 256, False, 520, None),
               # past three workgroups per CU: one block of activation rows, a half-empty one, three blocks
               ((4, 32), 32, 98400, 32, False, 5, None), ((8, 32), 32, 98400, 32, False, 33, None),
-              ((5, 32), 32, 33000, 64, False, 90, None)]
+              ((5, 32), 32, 33000, 64, False, 90, None),
+              # longer TQ columns take the GEMV's passes for two rounds ([900][1056], [400][640] above), then the tiles
+              ((4, 32), 32, 1000, 1056, False, 127, None), ((8, 16), 16, 480, 640, False, 289, None),
+              ((5, 32), 32, 256, 1024, False, 512, None), ((5, 32), 32, 256, 1024, False, 513, None)]
 
 
 @pytest.mark.parametrize("fmt,kb,rows,K,pair,m,strips", GEMM_CASES)
@@ -339,7 +342,7 @@ def test_gemv_many_rows_bit_exact(fmt, kb, rows, K, pair, m, strips):
     q, s, su = act_rows(O.gen_normal(5, 70 + m, m * K, 1.0).reshape(m, K), kb, pair)
     nstrips = (rows + 15) // 16
     s0, s1 = strips or (0, nstrips)
-    assert (s1 - s0) * ((q.shape[0] + 3) // 4) >= 7 * 256  # the tiles' range
+    assert (s1 - s0) * ((q.shape[0] + 3) // 4) >= 7 * 256  # the tiles' range (TQ of long columns: from 1920 or 2049)
     c0, c1 = 16 * s0, 16 * s1 if isinstance(fmt, tuple) else min(16 * s1, rows)
     ldy = 16 * nstrips + 3
     base = (np.arange(m * ldy, dtype=np.float32).reshape(m, ldy) % 97) * 0.25

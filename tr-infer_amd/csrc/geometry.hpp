@@ -141,6 +141,25 @@ inline bool gemm_narrow(uint64_t rb, uint64_t t32, uint32_t kb) {
     return c32 <= 3 || (kb == 16 ? 3 * c32 <= 4 * c64 : 2 * c32 <= 3 * c64);
 }
 
+// trk_gemv of many activation rows: its passes of four rows x strips are so many GEMV workgroups, four resident
+// per CU, so that it takes whole rounds of 1024; the tiles take as long for one row as for thirty-two.  The
+// tiles take over in the third round, before it where they beat two rounds: GGUF formats, whose GEMV decodes
+// more, and short columns, where the tiles' unpacking (dearer with more bits) is a smaller part.  us, GEMV /
+// tiles, at workgroups:
+//   GGUF from 1792: [4096][4096] Q6_K x 28 rows (1792) 89 / 76, [2560][2560] Q4_K x 48 (1920) 41 / 26;
+//   TQ [4096][3072] 1792 / 2048 / 2304: TQ4_32 26.5 / 28.8, 29.1 / 28.7, 33.7 / 29.0; TQ5_32 28.1 / 33.3, 30.5 /
+//   33.2, 35.1 / 33.3; TQ8_32 27.3 / 33.8, 30.1 / 33.6, 34.9 / 33.9; TQ5_16 48.7 / 52.9, 53.7 / 53.1, 61.0 / 53.0;
+//   [256][k] at 1792: TQ4_32 k = 1024 11.6 / 11.5, 1536 15.4 / 15.9; TQ5_32 768 10.8 / 10.4, 1024 12.1 / 13.0;
+//   TQ8_32 768 10.8 / 10.5, TQ8_16 512 11.3 / 11.5, 768 14.5 / 15.7;
+//   longer ones: [320][10240] TQ4_32 1920 82 / 89, 2080 101 / 89; TQ5_32 1920 87 / 104, 2320 113 / 104; TQ8_32 2060
+//   100 / 107, 2320 111 / 106.
+inline bool gemv_tiles(uint64_t workgroups, uint32_t tq, uint32_t k) {  // tq: 0 for GGUF, else bits << 8 | kb
+    const uint32_t bits = tq >> 8;
+    if (tq == 0 || k <= (bits == 4 ? 1024u : tq == 0x810 ? 512u : 768u)) return workgroups >= 1792;
+    if (bits == 4 && k <= 3072) return workgroups >= 1920;
+    return workgroups > (bits == 8 && k > 3072 ? 2303u : 2048u);
+}
+
 // Every invariant a call of m rows with kcap selections per token relies on; returns nullptr when
 // they hold, else what failed.  tq: the experts are TQ strips (k_tq.hip), not GGUF superblocks.
 inline const char* check_call(const Caps& c, uint32_t m, uint32_t kcap, bool tq = false) {

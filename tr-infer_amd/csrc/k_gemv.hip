@@ -541,14 +541,10 @@ static hipError_t gemv_go(const GemvArgs& g, uint32_t na, uint32_t gy, hipStream
 hipError_t launch_gemv(const Mat& w, uint32_t item, uint32_t s0, uint32_t s1, uint32_t kb, const int8_t* q,
                        const float* s, const int32_t* su, uint32_t m, int pair, float* y, uint32_t ldy,
                        const uint32_t* rows, int accumulate, hipStream_t st) {
-    // Many activation rows run as MFMA tiles once the GEMV would need seven workgroups per CU (a
-    // workgroup per strip and pass of four rows): below that its shorter K walk wins.  us, GEMV / tiles:
-    // [12288][2560] TQ4_32 x 8 (6 per CU) 22 / 25, x 16 (12) 35 / 25; [2560][640] TQ5_16 x 32 (5) 13 /
-    // 14; [4096][4096] Q6_K x 16 (4) 47 / 80, x 32 (8) 90 / 81; [24576][2048] Q4_K x 8 (12) 48 / 26
-    // A row map may repeat rows in an order of its own and stays here.
-    if (!rows && m > GV_NA && (uint64_t)(s1 - s0) * ((m + GV_NA - 1) / GV_NA) >= 7 * 256)
-        return launch_gemm(w, item, s0, s1, kb, q, s, su, m, pair, y, ldy, accumulate, st);
     const bool tq = fmt_is_tq(w.fmt);
+    // many activation rows as MFMA tiles; a row map may repeat rows in an order of its own and stays here
+    if (!rows && m > GV_NA && geo::gemv_tiles((uint64_t)(s1 - s0) * ((m + GV_NA - 1) / GV_NA), tq ? w.fmt : 0u, w.k))
+        return launch_gemm(w, item, s0, s1, kb, q, s, su, m, pair, y, ldy, accumulate, st);
     GemvArgs g;
     g.w = w.ptr + (size_t)item * w.stride;
     g.pitch = w.row_bytes;
