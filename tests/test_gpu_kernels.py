@@ -309,6 +309,19 @@ def test_gemv_few_rows_bit_exact(bits, kb, rows, K, pair, m, strips):
     gemv_check(to_dev(tq), tq, rows, K, (bits << 8) | kb, bits, kb, x, pair, strips)
 
 
+@pytest.mark.parametrize("kind,kb", [(4, 32), (4, 16), (5, 32), (5, 16), (6, 32), (6, 16)])
+@pytest.mark.parametrize("na", [1, 2, 4])
+def test_gemv_quads_two_workgroups_per_cu(kind, kb, na):
+    """The row quads' rule counts two of their workgroups per CU: registers and LDS leave room for them."""
+    import ctypes as C
+    torch_dev().zeros(1, device="cuda")
+    hip = C.CDLL("libamdhip64.so")
+    kernel = getattr(trmoe.lib(), f"_ZN3trk16gemv_quad_kernelILi{kind}ELi{kb}ELi{na}EEEvNS_8GemvArgsE")
+    n = C.c_int()
+    assert hip.hipOccupancyMaxActiveBlocksPerMultiprocessor(C.byref(n), C.cast(kernel, C.c_void_p), 512, C.c_size_t(0)) == 0
+    assert n.value >= 2
+
+
 # Enough (strip, pass) workgroups for the MFMA tiles: every codec, ragged row and activation tiles (the
 # last workgroup nearly empty), k short of a slice and past one, strip sub-ranges, pairs, accumulate;
 # 64-row workgroups past three of 32 rows per CU (m = 520 at 48 row blocks)

@@ -381,9 +381,10 @@ constexpr uint32_t GQ_T = 512;  // threads of gemv_quad_kernel
 // slice's loads in flight at once, and the chain's terms (m, u, dot, d * sx) are formed in phase 1, so
 // that a chain step is one 16-byte LDS read and two fmas.  Bound by that chain and the staging around it.
 // [320][10240] TQ8_32, us a call at 1 / 2 / 4 rows: 18.3 / 22.9 / 31.8 -> 11.2 / 12.7 / 15.5 (256 threads
-// instead of 512: 11.7 / 14.5 / 19.1).
+// instead of 512: 11.7 / 14.5 / 19.1).  At most 128 registers, or one workgroup fills a CU: one row of 5- and
+// 8-bit strips took 130 to 132, [2048][4096] TQ8_32 9.8 us against 7.3 now and 7.9 on a strip per workgroup.
 template <int GK, int KB, int NA>
-__global__ __launch_bounds__(GQ_T) void gemv_quad_kernel(GemvArgs g) {
+__global__ __launch_bounds__(GQ_T, 4) void gemv_quad_kernel(GemvArgs g) {
     using T = GvTQ<GK, KB>;
     constexpr uint32_t S = NA <= 2 ? 256 : 128, NU = S / (GQ_T / 4);  // blocks per slice, units per lane quad
     constexpr bool XSUM = GK == GK_TQ8;
