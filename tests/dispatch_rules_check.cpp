@@ -73,6 +73,16 @@ static void tiles() {
     for (auto& c : mfma) expect(gemv_tiles(c[0], c[1], c[2]), true, "gemv_tiles", c[0], c[1], c[2]);
 }
 
+// (rows x passes, activation rows a pass, bits, blocks a row): row quads from enough blocks
+static void quads() {
+    const unsigned strips[][4] = {{1024, 1, 4, 10}, {64, 2, 5, 16}, {1024, 1, 8, 32}, {1024, 2, 8, 20}, {320, 4, 8, 16}, {2048, 1, 5, 48},
+                                  {2048, 1, 8, 64}, {2048, 2, 8, 48}, {2048, 4, 4, 20}, {2064, 4, 4, 320}, {12288, 1, 5, 80}};
+    const unsigned quad[][4] = {{1024, 1, 4, 40}, {64, 2, 5, 40}, {1024, 1, 8, 48}, {1024, 2, 8, 40}, {320, 4, 8, 20}, {2048, 1, 5, 128},
+                                {2048, 1, 8, 128}, {2048, 2, 4, 80}, {2048, 4, 4, 40}, {320, 1, 8, 320}, {640, 2, 8, 320}};
+    for (auto& c : strips) expect(gemv_quads(c[0], c[1], c[2], c[3]), false, "gemv_quads", c[0], c[1], c[3]);
+    for (auto& c : quad) expect(gemv_quads(c[0], c[1], c[2], c[3]), true, "gemv_quads", c[0], c[1], c[3]);
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "router")) router();
@@ -80,6 +90,7 @@ int main(int argc, char** argv) {
     if (!std::strcmp(what, "grids")) grids();
     if (!std::strcmp(what, "gemm")) gemm();
     if (!std::strcmp(what, "tiles")) tiles();
+    if (!std::strcmp(what, "quads")) quads();
     if (!n || bad) return 1;
     std::printf("ok %d\n", n);
     return 0;

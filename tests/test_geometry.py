@@ -24,7 +24,7 @@ def test_launch_geometry_sweep():
         assert r.stdout.startswith("ok ") and int(r.stdout.split()[1]) > 100000
 
 
-@pytest.mark.parametrize("rule", ["router", "chunks", "grids", "gemm", "tiles"])
+@pytest.mark.parametrize("rule", ["router", "chunks", "grids", "gemm", "tiles", "quads"])
 def test_dispatch_rules_take_the_faster_form(rule):
     """tests/dispatch_rules_check.cpp: the rules that choose between two kernels, at sizes where both were timed."""
     with tempfile.TemporaryDirectory() as d:

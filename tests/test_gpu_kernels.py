@@ -292,13 +292,19 @@ def test_gemv_tq_bit_exact(bits, kb, rows, K, pair, m, strips):
     gemv_check(to_dev(tq), tq, rows, K, fmt, bits, kb, x, pair, strips)
 
 
-# Few TQ rows take four rows per workgroup (rows x passes of four up to 2048), more a strip per workgroup:
-# both sides of the line, slices of 256 blocks (128 from three activation rows) and one block past them
+# Few TQ rows of enough blocks take four rows per workgroup (rows x passes of four up to 2048; from 20 to 96 blocks
+# by those, the activation rows and the bits), others a strip per workgroup: both sides of the lines, slices of 256
+# blocks (128 from three activation rows) and one block past them
 GEMV_QUAD_CASES = [(4, 32, 2048, 320, False, 1, None), (4, 32, 2064, 320, False, 3, None),
                    (5, 32, 2064, 352, True, 1, None), (8, 32, 2064, 96, False, 2, None),
                    (4, 16, 2080, 80, False, 4, (1, 130)), (5, 16, 512, 4112, True, 1, (3, 32)),
                    (8, 32, 320, 10240, True, 1, None), (8, 32, 64, 4128, False, 4, None),
-                   (8, 16, 48, 2064, False, 3, (0, 2)), (4, 16, 1024, 4096, False, 8, None)]
+                   (8, 16, 48, 2064, False, 3, (0, 2)), (4, 16, 1024, 4096, False, 8, None),
+                   (4, 32, 256, 608, False, 1, None), (4, 32, 256, 640, False, 1, None),
+                   (8, 32, 96, 1248, True, 1, None), (8, 32, 96, 1280, True, 1, None), (8, 32, 96, 640, False, 3, None),
+                   (5, 16, 1040, 1008, False, 1, None), (5, 16, 1040, 1024, False, 2, None),
+                   (8, 16, 2048, 1520, False, 1, (0, 128)), (8, 16, 2048, 1536, False, 1, (0, 128)),
+                   (4, 16, 2048, 624, False, 4, None), (4, 16, 2048, 640, False, 4, None)]
 
 
 @pytest.mark.parametrize("bits,kb,rows,K,pair,m,strips", GEMV_QUAD_CASES)

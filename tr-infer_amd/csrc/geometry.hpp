@@ -141,6 +141,22 @@ inline bool gemm_narrow(uint64_t rb, uint64_t t32, uint32_t kb) {
     return c32 <= 3 || (kb == 16 ? 3 * c32 <= 4 * c64 : 2 * c32 <= 3 * c64);
 }
 
+// trk_gemv on TQ strips of few rows: four rows a workgroup (gemv_quad_kernel) or a strip's sixteen.  Row quads put
+// four times the workgroups on the GPU, two per CU at 2048 (row, pass) pairs, for staging that a strip does once:
+// they are ahead where a row has enough blocks, earlier while each has a CU of its own and with more activation
+// rows (more chains to share), later with 8 bits (the bytes summed besides).  us, strips / quads, at blocks:
+//   a CU each, 1024 rows x 1: TQ4_32 10 3.2 / 3.4, 20 3.6 / 3.6, 40 4.1 / 3.8, 80 5.8 / 4.5; TQ8_32 20 3.6 / 3.8, 40
+//   4.2 / 4.2, 64 5.0 / 4.6; 320 x 4: TQ8_32 10 4.1 / 4.7, 20 5.3 / 5.0, 40 6.6 / 5.3;
+//   two per CU, 2048 rows x 1: TQ5_32 20 3.7 / 4.4, 64 5.3 / 5.2, 128 8.1 / 6.7; TQ8_32 64 5.1 / 5.5, 128 7.9 / 7.3;
+//   x 4: TQ4_32 20 5.2 / 5.3, 40 6.5 / 5.7.  [320][10240] TQ8_32 at 1 / 2 / 4 rows 18.3 / 22.9 / 31.8 strips, 11.2 / 12.7
+//   / 15.5 quads; beyond 2048, [12288][2560] TQ5_32 x 2 11.3 / 28.5.
+// na: activation rows a pass (1, 2, 4).
+inline bool gemv_quads(uint64_t row_passes, uint32_t na, uint32_t bits, uint32_t blocks) {
+    if (row_passes > 2048) return false;
+    if (row_passes <= 1024) return blocks >= (bits == 8 && na < 4 ? 40u : 20u);
+    return blocks >= (na == 4 ? 40u : bits != 8 ? 64u : na == 2 ? 80u : 96u);
+}
+
 // trk_gemv of many activation rows: its passes of four rows x strips are so many GEMV workgroups, four resident
 // per CU, so that it takes whole rounds of 1024; the tiles take as long for one row as for thirty-two.  The
 // tiles take over in the third round, before it where they beat two rounds: GGUF formats, whose GEMV decodes

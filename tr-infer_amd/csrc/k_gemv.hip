@@ -522,9 +522,7 @@ template <int GK, int KB>
 static hipError_t gemv_go(const GemvArgs& g, uint32_t na, uint32_t gy, hipStream_t st) {
     const uint32_t n = g.r_hi - g.r_lo;
     if constexpr (GK >= GK_TQ4) {
-        // up to two such workgroups per CU.  us, strips / row quads at 2 rows: [2048][10240] TQ5_32 (512
-        // workgroups) 23.6 / 15.5, [1024][6400] 16.4 / 9.3; beyond, [12288][2560] 11.3 / 28.5
-        if ((uint64_t)n * gy <= 2048) {
+        if (geo::gemv_quads((uint64_t)n * gy, na, GvTQ<GK, KB>::BITS, g.nb)) {
             const dim3 grid(n / 4, gy);
             if (na <= 1)
                 gemv_quad_kernel<GK, KB, 1><<<grid, GQ_T, 0, st>>>(g);
