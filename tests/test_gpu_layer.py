@@ -149,6 +149,38 @@ def test_decode_one_launch_matches_three(policy):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("M,E,k", [(255, 1000, 3), (256, 24, 2), (512, 1024, 10), (513, 24, 2), (1024, 1000, 2),
+                                   (1025, 1024, 10), (1090, 513, 32)])
+def test_dispatch_arrays_by_chunks(M, E, k):
+    """The dispatch against a stable sort of its own selections, at the edges of its forms: one workgroup alone
+    (below 256 tokens), one round's masks, counted chunks kept (up to 16) or read again, two experts a thread."""
+    say(f"dispatch M={M} E={E} k={k}")
+    import torch
+    H = F = 256
+    W = trmoe.LayerWeights.generate(5, 0, H, E, F)
+    ctx = trmoe.Context(H, E, F, k, M)
+    x, out = torch.randn((M, H), device="cuda"), torch.empty((M, H), device="cuda")
+    lg = np.random.default_rng(M).standard_normal((M, E)).astype(np.float32)
+    lg[:, E // 2] += 3  # one long group
+    for _ in range(2):  # the second call finds the first one's arrays
+        ctx.forward(W, x, out, rlog=dev(lg))
+    ids = ctx.read(trmoe.WS_IDS, M * 32 * 4, np.uint32).reshape(M, 32)[:, :k]
+    w = ctx.read(trmoe.WS_W, M * 32 * 4, np.float32).reshape(M, 32)[:, :k]
+    tok, exp = np.repeat(np.arange(M), k), ids.reshape(-1)
+    order = np.lexsort((tok, exp))
+    ng, n_ent = ctx.read(trmoe.WS_NGROUPS, 16, np.uint32)[:2]
+    sizes = np.bincount(exp, minlength=E)
+    assert n_ent == M * k and ng == (sizes > 0).sum()
+    assert np.array_equal(ctx.read(trmoe.WS_ENT_TOK, 4 * n_ent, np.uint32), tok[order])
+    assert np.array_equal(ctx.read(trmoe.WS_ENT_EXP, 4 * n_ent, np.uint32), exp[order])
+    ent_w = ctx.read(trmoe.WS_ENT_W, 4 * n_ent, np.float32)
+    assert np.array_equal(ent_w.view(np.uint32), w.reshape(-1)[order].view(np.uint32))
+    gs = np.concatenate([[0], np.cumsum(sizes[sizes > 0])]).astype(np.uint32)
+    assert np.array_equal(ctx.read(trmoe.WS_GRP_START, 4 * (ng + 1), np.uint32), gs)
+    assert np.array_equal(ctx.read(trmoe.WS_GRP_EXP, 4 * ng, np.uint32), np.flatnonzero(sizes).astype(np.uint32))
+    ctx.close()
+
+
 @pytest.mark.parametrize("shape,M,k", [("small", 4, 4), ("small", 16, 4), ("small", 37, 6), ("full", 4, 10),
                                        ("full", 8, 10), ("full", 16, 10), ("small", 700, 3), ("small", 2200, 2),
                                        ("odd", 2100, 5)])
