@@ -37,16 +37,15 @@ __device__ __forceinline__ uint32_t load_ids(const Workspace& ws, uint32_t t, ui
     return ns;
 }
 
-// Single workgroup of DISPATCH_WAVES waves, one token per thread per round of DT tokens (ids and
-// weights stay in registers).  Per round each wave ORs its 64 tokens into a per-(wave, expert) lane
-// mask, so a token's rank within its expert is the popcount of the lower lanes' bits plus the
-// counts of the earlier waves and rounds: the reference's token-major order.  Expert starts,
-// group indices and work-item offsets come from one block-wide scan (a DPP scan per wave, then
+// Single workgroup of DISPATCH_WAVES waves.  Up to DT tokens it takes one per thread (ids and weights stay in
+// registers): each wave ORs its 64 tokens into a per-(wave, expert) lane mask, so a token's rank within its
+// expert is the popcount of the lower lanes' bits plus the counts of the earlier waves, the reference's
+// token-major order.  Beyond DT the counts per 64-token chunk come from count_kernel, in ws.doff.  Expert
+// starts, group indices and work-item offsets come from one block-wide scan (a DPP scan per wave, then
 // the wave totals).  kc4 = ceil(largest selection / 4).
-constexpr uint32_t DT = DISPATCH_WAVES * 64;  // tokens per round
-// split: leave the scatter to scatter_kernel (many workgroups) and store the per-(64-token chunk,
-// expert) first positions in ws.doff instead: from each chunk's counts (count_kernel's over several
-// rounds, one round's own masks) one prefix per expert over the chunks (no second pass over the tokens).
+constexpr uint32_t DT = DISPATCH_WAVES * 64;
+// split (always beyond DT): leave the scatter to scatter_kernel (many workgroups) and store the per-(64-token
+// chunk, expert) first positions in ws.doff: one prefix per expert over the chunks' counts.
 __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace ws, uint32_t m, uint32_t kc4,
                                                                        int split) {
     const uint32_t E = ws.E, tid = threadIdx.x;
@@ -57,39 +56,15 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
     uint32_t* run = cnt + E;                                                  // [E]
     uint32_t* off = run + E;                                                  // [W][E]
     uint32_t* wtot = off + DISPATCH_WAVES * E;                                // [W][5]
-    const uint32_t rounds = (m + DT - 1) / DT, nchunks = (m + 63) / 64;
+    const uint32_t nchunks = (m + 63) / 64;
     const uint32_t ept = (E + DT - 1) / DT;  // experts per thread in the scans (contiguous)
 
-    uint32_t id[K_MAX], ns = 0;
+    // Per-expert counts.  Up to 16 chunks a thread keeps its experts' counted ones (E <= 2 DT) for the prefix at
+    // the end: read again there, the launch was slower than masks at two selections per token (E = 512 x 600
+    // tokens 10.9 us against 10.2; 10.2 now, E = 128 x 10 x 600 12.2, 10.9 and 10.3)
+    uint32_t kept[2][16], id[K_MAX], ns = 0;
     float wt[K_MAX];
-    auto load_tok = [&](uint32_t r) {
-        const uint32_t t = r * DT + tid;
-        ns = t < m ? load_ids(ws, t, kc4, id) : 0u;
-        if (t < m) {
-#pragma unroll
-            for (uint32_t q = 0; q < K_MAX / 4; q++)
-                if (q < kc4) {
-                    const float4 v = reinterpret_cast<const float4*>(ws.w + (size_t)t * K_MAX)[q];
-                    wt[4 * q] = v.x; wt[4 * q + 1] = v.y; wt[4 * q + 2] = v.z; wt[4 * q + 3] = v.w;
-                }
-        }
-    };
-    auto build_masks = [&]() {  // ends with the masks complete
-        for (uint32_t i = tid; i < DISPATCH_WAVES * E; i += DT) masks[i] = 0ull;
-        __syncthreads();
-        uint32_t* mw = reinterpret_cast<uint32_t*>(masks + wv * E);
-#pragma unroll
-        for (uint32_t s = 0; s < K_MAX; s++)
-            if (s < ns) atomicOr(&mw[id[s] * 2 + (lane >> 5)], 1u << (lane & 31));
-        __syncthreads();
-    };
-
-    // pass 1: per-expert counts (over several rounds count_kernel left them per chunk in ws.doff).  Up to 16
-    // chunks a thread keeps its experts' (E <= 2 DT) for the prefix at the end: read again there, the launch
-    // was slower than the masks it replaces at two selections per token (E = 512 x 600 tokens 10.9 us
-    // against 10.2; 10.2 now, E = 128 x 10 x 600 12.2, 10.9 and 10.3)
-    uint32_t kept[2][16];
-    if (split && rounds > 1) {
+    if (m > DT) {
 #pragma unroll
         for (uint32_t i = 0; i < 2; i++) {
             const uint32_t e = tid + DT * i;
@@ -107,17 +82,27 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
             cnt[e] = c;
         }
     } else {
-        for (uint32_t e = tid; e < E; e += DT) cnt[e] = 0;
-    }
-    for (uint32_t r = 0; r < (split && rounds > 1 ? 0u : rounds); r++) {
-        load_tok(r);
-        build_masks();
+        if (tid < m) {
+            ns = load_ids(ws, tid, kc4, id);
+#pragma unroll
+            for (uint32_t q = 0; q < K_MAX / 4; q++)
+                if (q < kc4) {
+                    const float4 v = reinterpret_cast<const float4*>(ws.w + (size_t)tid * K_MAX)[q];
+                    wt[4 * q] = v.x; wt[4 * q + 1] = v.y; wt[4 * q + 2] = v.z; wt[4 * q + 3] = v.w;
+                }
+        }
+        for (uint32_t i = tid; i < DISPATCH_WAVES * E; i += DT) masks[i] = 0ull;
+        __syncthreads();
+        uint32_t* mw = reinterpret_cast<uint32_t*>(masks + wv * E);
+#pragma unroll
+        for (uint32_t s = 0; s < K_MAX; s++)
+            if (s < ns) atomicOr(&mw[id[s] * 2 + (lane >> 5)], 1u << (lane & 31));
+        __syncthreads();
         for (uint32_t e = tid; e < E; e += DT) {
-            uint32_t c = cnt[e];
+            uint32_t c = 0;
             for (uint32_t w = 0; w < DISPATCH_WAVES; w++) c += popc64(masks[w * E + e]);
             cnt[e] = c;
         }
-        if (rounds > 1) __syncthreads();
     }
     __syncthreads();
 
@@ -195,17 +180,7 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
     }
     __syncthreads();
 
-    if (split && rounds == 1) {  // one round: the chunk counts are the masks still in LDS
-        for (uint32_t e = tid; e < E; e += DT) {
-            uint32_t o = run[e];
-            for (uint32_t w = 0; w < DISPATCH_WAVES && w < nchunks; w++) {
-                ws.doff[(size_t)w * E + e] = o;
-                o += popc64(masks[w * E + e]);
-            }
-        }
-        return;
-    }
-    if (split) {  // the chunk counts become each chunk's first position per expert
+    if (m > DT) {  // the chunk counts become each chunk's first position per expert
 #pragma unroll
         for (uint32_t i = 0; i < 2; i++) {
             const uint32_t e = tid + DT * i;
@@ -225,35 +200,36 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
         }
         return;
     }
-    // pass 2: scatter (the single-round case reuses the masks and the registers of pass 1)
-    const unsigned long long below = lane ? ((1ull << lane) - 1ull) : 0ull;
-    for (uint32_t r = 0; r < rounds; r++) {
-        if (rounds > 1) {
-            load_tok(r);
-            build_masks();
-        }
+    if (split) {  // the chunk counts are the masks still in LDS
         for (uint32_t e = tid; e < E; e += DT) {
             uint32_t o = run[e];
-            for (uint32_t w = 0; w < DISPATCH_WAVES; w++) {
-                off[w * E + e] = o;
+            for (uint32_t w = 0; w < DISPATCH_WAVES && w < nchunks; w++) {
+                ws.doff[(size_t)w * E + e] = o;
                 o += popc64(masks[w * E + e]);
             }
-            run[e] = o;
         }
-        __syncthreads();
-        const uint32_t t = r * DT + tid;
-#pragma unroll
-        for (uint32_t s = 0; s < K_MAX; s++)
-            if (s < ns) {
-                const uint32_t e = id[s];
-                const uint32_t pos = off[wv * E + e] + popc64(masks[wv * E + e] & below);
-                ws.ent_tok[pos] = t;
-                ws.ent_w[pos] = wt[s];
-                ws.ent_exp[pos] = e;
-                ws.ent_of[(size_t)t * K_MAX + s] = pos;
-            }
-        if (rounds > 1) __syncthreads();
+        return;
     }
+    // the scatter
+    const unsigned long long below = lane ? ((1ull << lane) - 1ull) : 0ull;
+    for (uint32_t e = tid; e < E; e += DT) {
+        uint32_t o = run[e];
+        for (uint32_t w = 0; w < DISPATCH_WAVES; w++) {
+            off[w * E + e] = o;
+            o += popc64(masks[w * E + e]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t s = 0; s < K_MAX; s++)
+        if (s < ns) {
+            const uint32_t e = id[s];
+            const uint32_t pos = off[wv * E + e] + popc64(masks[wv * E + e] & below);
+            ws.ent_tok[pos] = tid;
+            ws.ent_w[pos] = wt[s];
+            ws.ent_exp[pos] = e;
+            ws.ent_of[(size_t)tid * K_MAX + s] = pos;
+        }
 }
 
 // The entries of every expert in one 64-token chunk (a workgroup per chunk), into ws.doff.
@@ -454,9 +430,10 @@ hipError_t launch_dispatch(const Workspace& ws, uint32_t m, uint32_t kcap, hipSt
     // from a few hundred tokens on, one workgroup's scattered stores dominate: spread them
     const int split = geo::dispatch_split(m) ? 1 : 0;
     if (split && geo::doff_elems(m, ws.E) > geo::doff_elems(ws.m_max, ws.E)) return hipErrorInvalidValue;
-    // over several rounds of DT tokens the counts come from a workgroup per chunk: one workgroup building
-    // every round's masks took 30 of 41 us at 3,072 tokens (41 -> 5 + 12 us); one round keeps its masks
-    if (split && m > DT) count_kernel<<<geo::chunks(m), 256, E * 4, st>>>(ws, m, (kcap + 3) / 4);
+    if (m > DT && !split) return hipErrorInvalidValue;
+    // beyond DT tokens the counts come from a workgroup per chunk: one workgroup building every DT tokens' masks
+    // took 27 us of dispatch at 3,072 tokens (17 now; E = 512, k = 10); up to DT it keeps its masks
+    if (m > DT) count_kernel<<<geo::chunks(m), 256, E * 4, st>>>(ws, m, (kcap + 3) / 4);
     dispatch_kernel<<<1, DT, lds, st>>>(ws, m, (kcap + 3) / 4, split);
     if (split) scatter_kernel<<<geo::chunks(m), 64, E * 12, st>>>(ws, m, (kcap + 3) / 4);
     return hipGetLastError();
