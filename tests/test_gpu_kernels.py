@@ -143,6 +143,33 @@ def test_router_mfma_chunks_bit_exact(m, E, H):
     assert np.array_equal(host(sh).view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("m,E,H", [(512, 512, 256), (200, 512, 192), (1030, 64, 384), (40, 64, 256)])
+def test_router_gemm_special_values_bit_exact(m, E, H):
+    """Denormal inputs, products and sums, signed zeros, overflow and infinities through the outer products (and
+    the VALU tiles): the bits of the oracle's fma chains, NaN where it has NaN."""
+    say(f"router special values m={m} E={E} H={H}")
+    rng = np.random.default_rng(m)
+    scale = np.float32(2.0) ** rng.integers(-40, 30, (m, 1)).astype(np.float32)
+    x = (rng.standard_normal((m, H)).astype(np.float32) * scale)
+    router = rng.standard_normal((E, H)).astype(np.float32)
+    x[0::8] *= np.float32(2.0 ** -60)   # products in the denormal range
+    router[0::4] *= np.float32(2.0 ** -60)
+    x[1::8] = (rng.integers(0, 1 << 23, x[1::8].shape).astype(np.uint32) | (rng.integers(0, 2, x[1::8].shape).astype(np.uint32) << 31)).view(np.float32)
+    x[2::8] = np.where(rng.random(x[2::8].shape) < 0.5, np.float32(-0.0), x[2::8])
+    x[3::8, 5] = np.float32(3e38)       # overflow inside a chain
+    router[1::4, 5] = np.float32(3e38)
+    x[4::8, 7] = np.inf
+    x[5::8, 9], x[5::8, 25] = np.inf, -np.inf  # one chain, or two that meet in the tree
+    router[2::4, 9] = 0.0               # inf * 0
+    with np.errstate(all="ignore"):
+        want = O.gemm_f32_nt(x, router)
+    got = host(trmoe.router_logits(to_dev(router), to_dev(x), gemm_order=True)[0])
+    nan = np.isnan(want)
+    assert nan.any() and np.isinf(want).any() and ((np.abs(want) < 1e-38) & (want != 0)).any()
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+
+
 @pytest.mark.parametrize("n,H", [(32 * 2897, 64), (23200, 16)])
 def test_router_more_tiles_than_one_grid_row(n, H):
     """n x n logits whose tiles pass 2^32 threads (32 x 32 of 512 threads, 34 GB; 16 x 2 of 256): every sampled
@@ -312,6 +339,23 @@ def test_gemv_few_rows_bit_exact(bits, kb, rows, K, pair, m, strips):
     say(f"gemv quads bits={bits} kb={kb} rows={rows} K={K} pair={pair} m={m} strips={strips}")
     tq = random_tq(9 + bits + kb + m, rows, K, bits, kb)
     x = O.gen_normal(4, 80 + m, m * K, 1.0).reshape(m, K)
+    gemv_check(to_dev(tq), tq, rows, K, (bits << 8) | kb, bits, kb, x, pair, strips)
+
+
+# TQ strips that stay a workgroup per strip (64 rows a workgroup from 65,536), also with a row map: more rows than
+# the quads take, several passes of four activation rows (the last one partial), several slices of blocks
+GEMV_STRIP_CASES = [(5, 32, 2064, 2592, False, 7, None), (8, 32, 2064, 2080, True, 3, None), (8, 16, 2080, 1104, False, 9, None),
+                    (4, 16, 2064, 2064, False, 4, None), (5, 16, 2096, 1040, True, 2, None), (4, 32, 2064, 4128, False, 1, None),
+                    (4, 32, 65552, 1056, False, 3, None), (8, 32, 65536, 1056, False, 1, None),
+                    (5, 16, 65552, 560, True, 1, (0, 4097))]
+
+
+@pytest.mark.parametrize("bits,kb,rows,K,pair,m,strips", GEMV_STRIP_CASES)
+def test_gemv_strips_bit_exact(bits, kb, rows, K, pair, m, strips):
+    say(f"gemv strips bits={bits} kb={kb} rows={rows} K={K} pair={pair} m={m} strips={strips}")
+    assert rows > 2048 and (rows // 16) * ((m * (2 if pair else 1) + 3) // 4) < (1792 if m > 4 else 1 << 32)
+    tq = random_tq(13 + bits + kb + m, rows, K, bits, kb)
+    x = O.gen_normal(4, 90 + m, m * K, 1.0).reshape(m, K)
     gemv_check(to_dev(tq), tq, rows, K, (bits << 8) | kb, bits, kb, x, pair, strips)
 
 

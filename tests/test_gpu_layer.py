@@ -185,7 +185,7 @@ def test_dispatch_arrays_by_chunks(M, E, k):
                                        ("full", 8, 10), ("full", 16, 10), ("small", 700, 3), ("small", 2200, 2),
                                        ("odd", 2100, 5)])
 def test_batch_layer_and_dispatch(shape, M, k):
-    # M = 700: the split (parallel) scatter; M = 2200: three rounds of 1024 tokens, 35 chunks;
+    # M = 700: the split (parallel) scatter; M = 2200: counted chunks, 35 of them;
     # from M = 2048 the gate/up runs item pairs of one expert as 32-row tiles (odd: 3 superblocks)
     say(f"batch layer {shape} M={M} k={k}")
     L, orc, W = layer(shape, **{"small": SMALL, "full": FULL, "odd": ODD}[shape])
