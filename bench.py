@@ -533,7 +533,8 @@ def bench_gemv(args, dev, stream, trmoe, torch, np):
         ach = nbytes / (us * 1e-6) / 1e9
         res[name] = {"rows": rows, "k": k, "fmt": f"TQ{fmt >> 8}_{fmt & 0xff}", "MB": round(mb / 1e6, 2),
                      "us": round(us, 2), "GBps": round(ach, 1),
-                     "roofline": {"bound": "hbm", "kernel": "gemv_rows_kernel", "achieved": round(ach, 1),
+                     "roofline": {"bound": "hbm", "kernel": "gemv_quad_kernel" if rows <= 2048 else "gemv_rows_kernel",
+                                  "achieved": round(ach, 1),
                                   "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                                   "traffic": None, "alg_bytes_per_launch": int(nbytes), "avg_launch_us": round(us, 2)},
                      "copies": copies, "steps": steps}

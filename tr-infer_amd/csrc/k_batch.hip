@@ -46,6 +46,8 @@ __device__ __forceinline__ uint32_t load_ids(const Workspace& ws, uint32_t t, ui
 constexpr uint32_t DT = DISPATCH_WAVES * 64;
 // split (always beyond DT): leave the scatter to scatter_kernel (many workgroups) and store the per-(64-token
 // chunk, expert) first positions in ws.doff: one prefix per expert over the chunks' counts.
+// COUNTED: beyond DT, a kernel of its own (both forms' code and registers in one: 4.6 -> 5.3 us at 37 tokens x 2).
+template <bool COUNTED>
 __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace ws, uint32_t m, uint32_t kc4,
                                                                        int split) {
     const uint32_t E = ws.E, tid = threadIdx.x;
@@ -62,9 +64,9 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
     // Per-expert counts.  Up to 16 chunks a thread keeps its experts' counted ones (E <= 2 DT) for the prefix at
     // the end: read again there, the launch was slower than masks at two selections per token (E = 512 x 600
     // tokens 10.9 us against 10.2; 10.2 now, E = 128 x 10 x 600 12.2, 10.9 and 10.3)
-    uint32_t kept[2][16], id[K_MAX], ns = 0;
-    float wt[K_MAX];
-    if (m > DT) {
+    [[maybe_unused]] uint32_t kept[2][16], id[K_MAX], ns = 0;
+    [[maybe_unused]] float wt[K_MAX];
+    if constexpr (COUNTED) {
 #pragma unroll
         for (uint32_t i = 0; i < 2; i++) {
             const uint32_t e = tid + DT * i;
@@ -95,8 +97,11 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
         __syncthreads();
         uint32_t* mw = reinterpret_cast<uint32_t*>(masks + wv * E);
 #pragma unroll
-        for (uint32_t s = 0; s < K_MAX; s++)
-            if (s < ns) atomicOr(&mw[id[s] * 2 + (lane >> 5)], 1u << (lane & 31));
+        for (uint32_t q = 0; q < K_MAX / 4; q++)  // kc4 is uniform: the slots past it cost a scalar branch per four
+            if (q < kc4)
+#pragma unroll
+                for (uint32_t s = 4 * q; s < 4 * q + 4; s++)
+                    if (s < ns) atomicOr(&mw[id[s] * 2 + (lane >> 5)], 1u << (lane & 31));
         __syncthreads();
         for (uint32_t e = tid; e < E; e += DT) {
             uint32_t c = 0;
@@ -180,7 +185,7 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
     }
     __syncthreads();
 
-    if (m > DT) {  // the chunk counts become each chunk's first position per expert
+    if constexpr (COUNTED) {  // the chunk counts become each chunk's first position per expert
 #pragma unroll
         for (uint32_t i = 0; i < 2; i++) {
             const uint32_t e = tid + DT * i;
@@ -198,38 +203,41 @@ __global__ __launch_bounds__(DISPATCH_WAVES * 64) void dispatch_kernel(Workspace
                     }
             }
         }
-        return;
-    }
-    if (split) {  // the chunk counts are the masks still in LDS
+    } else {
+        if (split) {  // the chunk counts are the masks still in LDS
+            for (uint32_t e = tid; e < E; e += DT) {
+                uint32_t o = run[e];
+                for (uint32_t w = 0; w < DISPATCH_WAVES && w < nchunks; w++) {
+                    ws.doff[(size_t)w * E + e] = o;
+                    o += popc64(masks[w * E + e]);
+                }
+            }
+            return;
+        }
+        // the scatter
+        const unsigned long long below = lane ? ((1ull << lane) - 1ull) : 0ull;
         for (uint32_t e = tid; e < E; e += DT) {
             uint32_t o = run[e];
-            for (uint32_t w = 0; w < DISPATCH_WAVES && w < nchunks; w++) {
-                ws.doff[(size_t)w * E + e] = o;
+            for (uint32_t w = 0; w < DISPATCH_WAVES; w++) {
+                off[w * E + e] = o;
                 o += popc64(masks[w * E + e]);
             }
         }
-        return;
-    }
-    // the scatter
-    const unsigned long long below = lane ? ((1ull << lane) - 1ull) : 0ull;
-    for (uint32_t e = tid; e < E; e += DT) {
-        uint32_t o = run[e];
-        for (uint32_t w = 0; w < DISPATCH_WAVES; w++) {
-            off[w * E + e] = o;
-            o += popc64(masks[w * E + e]);
-        }
-    }
-    __syncthreads();
+        __syncthreads();
 #pragma unroll
-    for (uint32_t s = 0; s < K_MAX; s++)
-        if (s < ns) {
-            const uint32_t e = id[s];
-            const uint32_t pos = off[wv * E + e] + popc64(masks[wv * E + e] & below);
-            ws.ent_tok[pos] = tid;
-            ws.ent_w[pos] = wt[s];
-            ws.ent_exp[pos] = e;
-            ws.ent_of[(size_t)tid * K_MAX + s] = pos;
-        }
+        for (uint32_t q = 0; q < K_MAX / 4; q++)
+            if (q < kc4)
+#pragma unroll
+                for (uint32_t s = 4 * q; s < 4 * q + 4; s++)
+                    if (s < ns) {
+                        const uint32_t e = id[s];
+                        const uint32_t pos = off[wv * E + e] + popc64(masks[wv * E + e] & below);
+                        ws.ent_tok[pos] = tid;
+                        ws.ent_w[pos] = wt[s];
+                        ws.ent_exp[pos] = e;
+                        ws.ent_of[(size_t)tid * K_MAX + s] = pos;
+                    }
+    }
 }
 
 // The entries of every expert in one 64-token chunk (a workgroup per chunk), into ws.doff.
@@ -433,8 +441,12 @@ hipError_t launch_dispatch(const Workspace& ws, uint32_t m, uint32_t kcap, hipSt
     if (m > DT && !split) return hipErrorInvalidValue;
     // beyond DT tokens the counts come from a workgroup per chunk: one workgroup building every DT tokens' masks
     // took 27 us of dispatch at 3,072 tokens (17 now; E = 512, k = 10); up to DT it keeps its masks
-    if (m > DT) count_kernel<<<geo::chunks(m), 256, E * 4, st>>>(ws, m, (kcap + 3) / 4);
-    dispatch_kernel<<<1, DT, lds, st>>>(ws, m, (kcap + 3) / 4, split);
+    if (m > DT) {
+        count_kernel<<<geo::chunks(m), 256, E * 4, st>>>(ws, m, (kcap + 3) / 4);
+        dispatch_kernel<true><<<1, DT, lds, st>>>(ws, m, (kcap + 3) / 4, split);
+    } else {
+        dispatch_kernel<false><<<1, DT, lds, st>>>(ws, m, (kcap + 3) / 4, split);
+    }
     if (split) scatter_kernel<<<geo::chunks(m), 64, E * 12, st>>>(ws, m, (kcap + 3) / 4);
     return hipGetLastError();
 }
