@@ -2,7 +2,8 @@
 // types), shared by the launchers, the workspace sizing of trk_create and a CPU-only check that
 // sweeps shapes (tests/geometry_check.cpp).  Every grid a launcher builds and every workspace
 // extent a kernel indexes is computed here, so a grid that addresses strips past F or a buffer
-// sized below what a dispatch writes shows up on the host, without a GPU.
+// sized below what a dispatch writes shows up on the host, without a GPU.  The rules that choose between
+// two kernels by size are here too (tests/dispatch_rules_check.cpp: at sizes where both were timed).
 #pragma once
 
 #include <stdint.h>

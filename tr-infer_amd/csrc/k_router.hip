@@ -312,8 +312,8 @@ __global__ __launch_bounds__(256) void router_gemm_kernel(const float* __restric
 }
 
 // The same gemm_f32_nt order on the matrix cores.  v_mfma_f32_16x16x1f32 is 4 independent 16x16 outer
-// products with accumulate, each element one fma rounded once (the same bits as v_fma_f32, checked on
-// gfx950 over random bit patterns, denormals and infinities).  Lane l = 16 b + r gives block b its
+// products with accumulate, each element one fma rounded once (the same bits as v_fma_f32, at denormals,
+// overflow and infinities too).  Lane l = 16 b + r gives block b its
 // A value x[token r][k] and its B value w[expert r][k]; with k = 16 s + 4 b + c the instructions
 // c = 0..3 of step s run the sixteen chains j = 4 b + c of a 16-token x 16-expert tile.  Two waves share
 // a tile, two c each, so a lane's operands of a step are one 8-byte LDS read each of x and w for two
@@ -324,8 +324,8 @@ __global__ __launch_bounds__(256) void router_gemm_kernel(const float* __restric
 // Up to about 512 rows the time is a workgroup's walk over its chunks (H = 2048: 0.5 us a chunk beside
 // its MFMAs, hence the wide chunks); at 3,072 the tiles' reads of x and router (0.8 GB through L2).
 // E = 512, H = 2048 x 512 rows 26.5 -> 21.2 us, H = 2560 x 500 rows (VALU tiles before) 40.2 -> 26.3 us
-// against v_mfma_f32_4x4x1f32 tiles (eight 4-byte reads for sixteen instructions).  Where it runs:
-// geo::router_on_mfma.
+// against v_mfma_f32_4x4x1f32 tiles (eight 4-byte reads for sixteen instructions), launched repeatedly with
+// x's quantisation beside the tiles (the tiles alone 19.0 and 22.9).  Where it runs: geo::router_on_mfma.
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 template <int KC>
