@@ -493,3 +493,41 @@ def test_swiglu_and_rmsnorm_bit_exact():
     yn = host(trmoe.rmsnorm(to_dev(x), to_dev(w), 1e-6))
     want = np.stack([O.rmsnorm(x[i], w, 1e-6) for i in range(2)])
     assert np.array_equal(yn.view(np.uint32), want.view(np.uint32))
+
+
+def test_row_and_element_kernels_past_one_grid_row():
+    """swiglu, add, rmsnorm, route and the normal generator past 2^32 threads: the last elements and rows as a call
+    of their own gives them (swiglu's scalar tail is the whole array's)."""
+    torch = torch_dev()
+    if torch.cuda.mem_get_info()[0] < 80 << 30:
+        pytest.skip("needs 60 GB of free memory")
+    n = (1 << 32) + 16 * 1000
+    cuts = [slice(0, 4096), slice(n // 2, n // 2 + 4096), slice(n - 4096, n)]
+    say("swiglu, add of 2^32 elements")
+    part = torch.randn(1 << 20, device="cuda")
+    g = part.repeat(n // (1 << 20) + 1)[:n]
+    y = torch.empty(n, device="cuda")
+    trmoe.check(trmoe.lib().trk_swiglu(g.data_ptr(), g.data_ptr(), y.data_ptr(), n, None))
+    for c in cuts:
+        one = trmoe.swiglu(g[c].clone(), g[c].clone())
+        assert torch.equal(y[c].view(torch.int32), one.view(torch.int32)), c
+    trmoe.check(trmoe.lib().trk_add_inplace(y.data_ptr(), g.data_ptr(), n, None))
+    for c in cuts:
+        one = trmoe.swiglu(g[c].clone(), g[c].clone()) + g[c]
+        assert torch.equal(y[c].view(torch.int32), one.view(torch.int32)), c
+    say("rmsnorm, route of 2^26 rows")
+    m = (1 << 26) + 50
+    x = g[:4 * m].view(m, 4)
+    out = trmoe.rmsnorm(x, None, 1e-6)
+    ids, w, k = trmoe.route(x, 2)
+    for r in (0, m // 2, m - 10, m - 1):
+        assert torch.equal(out[r], trmoe.rmsnorm(x[r:r + 1].clone(), None, 1e-6)[0]), r
+        i1, w1, k1 = trmoe.route(x[r:r + 1].clone(), 2)
+        assert int(k[r]) == 2 and torch.equal(ids[r], i1[0]) and torch.equal(w[r], w1[0]), r
+    del g, y, out, ids, w, k, x
+    say("2^32 normals")
+    z = trmoe.gen_normal(7, 3, n)
+    assert torch.isfinite(z[n - 4096:]).all() and (z[n - 4096:] != z[n - (1 << 32) - 4096:n - (1 << 32)]).any()
+    assert 0.9 < float(z[n - 4096:].std()) < 1.1 and 0.9 < float(z[n // 2:n // 2 + 4096].std()) < 1.1
+    del z
+    torch.cuda.empty_cache()

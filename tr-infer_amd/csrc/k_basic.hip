@@ -93,22 +93,28 @@ hipError_t launch_quantize(const float* x, uint32_t m, uint32_t k, uint32_t kb, 
 // tail.
 __global__ void swiglu_kernel(const float* __restrict__ g, const float* __restrict__ u, float* __restrict__ y,
                               size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    size_t i = (size_t)run_id() * blockDim.x + threadIdx.x;
     if (i >= n) return;
     size_t body = n / 16 * 16;
     float gv = g[i];
     y[i] = (i < body ? silu512(gv) : gv * sigmoid_libm(gv)) * u[i];
 }
 
+// the launches of a thread per element or a wave per row: workgroups past 2^32 threads as rows of y
+static dim3 run_grid(size_t workgroups) {
+    const geo::Grid2 g = geo::grid_run(workgroups, 256);
+    return dim3(g.x, g.y);
+}
+
 hipError_t launch_swiglu(const float* g, const float* u, float* y, size_t n, hipStream_t st) {
-    swiglu_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(g, u, y, n);
+    swiglu_kernel<<<run_grid((n + 255) / 256), 256, 0, st>>>(g, u, y, n);
     return hipGetLastError();
 }
 
 // rmsnorm (elem.rs:255-262) with sumsq (elem.rs:224-252) in the dot order: one wave per row.
 __global__ void rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w, float eps, uint32_t m,
                                uint32_t n, float* __restrict__ y) {
-    uint32_t row = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
+    uint32_t row = run_id() * (blockDim.x / WAVE) + threadIdx.x / WAVE;
     uint32_t lane = threadIdx.x % WAVE;
     if (row >= m) return;
     const float* xr = x + (size_t)row * n;
@@ -130,17 +136,17 @@ __global__ void rmsnorm_kernel(const float* __restrict__ x, const float* __restr
 
 hipError_t launch_rmsnorm(const float* x, const float* w, float eps, uint32_t m, uint32_t n, float* y,
                           hipStream_t st) {
-    rmsnorm_kernel<<<(m + 3) / 4, 256, 0, st>>>(x, w, eps, m, n, y);
+    rmsnorm_kernel<<<run_grid(((size_t)m + 3) / 4), 256, 0, st>>>(x, w, eps, m, n, y);
     return hipGetLastError();
 }
 
 __global__ void add_kernel(float* __restrict__ y, const float* __restrict__ a, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    size_t i = (size_t)run_id() * blockDim.x + threadIdx.x;
     if (i < n) y[i] = y[i] + a[i];
 }
 
 hipError_t launch_add(float* y, const float* a, size_t n, hipStream_t st) {
-    add_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(y, a, n);
+    add_kernel<<<run_grid((n + 255) / 256), 256, 0, st>>>(y, a, n);
     return hipGetLastError();
 }
 
@@ -242,7 +248,7 @@ hipError_t launch_gen_gguf(uint32_t fmt, uint64_t seed, uint64_t stream0, uint64
 }
 
 __global__ void gen_normal_kernel(uint64_t key, size_t n, double sigma, float* out) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    size_t i = (size_t)run_id() * blockDim.x + threadIdx.x;
     if (i >= n) return;
     uint64_t a = rng_u64(key, 2 * i), b = rng_u64(key, 2 * i + 1);
     double u1 = ((double)(a >> 11) + 1.0) * (1.0 / 9007199254740992.0);
@@ -260,7 +266,7 @@ hipError_t launch_gen_normal(uint64_t seed, uint64_t stream_id, size_t n, double
         return z ^ (z >> 31);
     };
     uint64_t key = hmix(seed ^ hmix(stream_id));
-    gen_normal_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(key, n, sigma, out);
+    gen_normal_kernel<<<run_grid((n + 255) / 256), 256, 0, st>>>(key, n, sigma, out);
     return hipGetLastError();
 }
 

@@ -525,7 +525,7 @@ __global__ __launch_bounds__(256) void route_kernel(const float* __restrict__ lo
     __shared__ uint2 cand[4][ROUTE_CAND];
     extern __shared__ float ex_all[];  // [4][E] for MassBasis::All
     const uint32_t wv = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    const uint32_t row = blockIdx.x * 4 + wv;
+    const uint32_t row = run_id() * 4 + wv;
     if (row >= m) return;
     const uint32_t n = route_row<NJ>(logits + (size_t)row * E, E, k, pol, lane, cand[wv], ex_all + (size_t)wv * E,
                                      ids + (size_t)row * K_MAX, wout + (size_t)row * K_MAX);
@@ -541,10 +541,11 @@ __global__ __launch_bounds__(256) void route_kernel(const float* __restrict__ lo
 hipError_t launch_route(const float* logits, uint32_t m, uint32_t E, uint32_t k, Policy pol, uint32_t* ids,
                         float* w, uint32_t* n_sel, unsigned long long* stats, hipStream_t st) {
     const size_t lds = (pol.enabled && pol.basis == TRK_BASIS_ALL) ? (size_t)4 * E * sizeof(float) : 0;
+    const geo::Grid2 g = geo::grid_run(((uint64_t)m + 3) / 4, 256);
     if (E <= 512)
-        route_kernel<8><<<(m + 3) / 4, 256, lds, st>>>(logits, m, E, k, pol, ids, w, n_sel, stats);
+        route_kernel<8><<<dim3(g.x, g.y), 256, lds, st>>>(logits, m, E, k, pol, ids, w, n_sel, stats);
     else
-        route_kernel<16><<<(m + 3) / 4, 256, lds, st>>>(logits, m, E, k, pol, ids, w, n_sel, stats);
+        route_kernel<16><<<dim3(g.x, g.y), 256, lds, st>>>(logits, m, E, k, pol, ids, w, n_sel, stats);
     return hipGetLastError();
 }
 
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(256) void mass_profile_kernel(const float* __restri
     __shared__ float top_w[4][K_MAX];
     extern __shared__ float ex_all[];  // [4][E]
     const uint32_t wv = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    const uint32_t row = blockIdx.x * 4 + wv;
+    const uint32_t row = run_id() * 4 + wv;
     if (row >= m) return;
     const float* lg = logits + (size_t)row * E;
     const uint32_t kk = E < (uint32_t)K_MAX ? E : (uint32_t)K_MAX;
@@ -595,10 +596,11 @@ __global__ __launch_bounds__(256) void mass_profile_kernel(const float* __restri
 
 hipError_t launch_mass_profile(const float* logits, uint32_t m, uint32_t E, unsigned long long* prof, hipStream_t st) {
     const size_t lds = (size_t)4 * E * sizeof(float);
+    const geo::Grid2 g = geo::grid_run(((uint64_t)m + 3) / 4, 256);
     if (E <= 512)
-        mass_profile_kernel<8><<<(m + 3) / 4, 256, lds, st>>>(logits, m, E, prof);
+        mass_profile_kernel<8><<<dim3(g.x, g.y), 256, lds, st>>>(logits, m, E, prof);
     else
-        mass_profile_kernel<16><<<(m + 3) / 4, 256, lds, st>>>(logits, m, E, prof);
+        mass_profile_kernel<16><<<dim3(g.x, g.y), 256, lds, st>>>(logits, m, E, prof);
     return hipGetLastError();
 }
 
